@@ -56,12 +56,17 @@ namespace {
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// Offset of the scratch in a workspace's buffer, on a 128-byte line.
+size_t work_offset(int n, int nT) {
+  return ((size_t)n * nT * 4096 + ((size_t)n * nT + 1) + 1 + 4096 + 15) & ~(size_t)15;
+}
+
 size_t ws_doubles(int n, int b, int a, size_t* work_out) {
   const int nT = (b + 63) / 64;
-  // scratch for solve / selected inversion: 3 b x b blocks + arrow temporaries
-  const size_t work = 3 * (size_t)b * b + 4 * (size_t)a * b + 2 * (size_t)a * a + 64;
+  // scratch of the sweeps: hand-over vectors, or the arrow's partial sums
+  const size_t work = std::max(3 * (size_t)b * b + 4 * (size_t)a * b + 2 * (size_t)a * a + 64, bta::sweep_doubles(n, b));
   if (work_out) *work_out = work;
-  return (size_t)n * nT * 4096 + ((size_t)n * nT + 1) + 1 + 4096 + work;
+  return work_offset(n, nT) + work;
 }
 
 // Run `enqueue` either directly on `st` or through a cached hipGraph.
@@ -184,12 +189,16 @@ int bta_ws_create(int device, int n, int b, int a, int flags, bta_ws_t* out) {
   w.logpart = w.winv + (size_t)n * w.nT * 4096;
   w.logdet = w.logpart + (size_t)n * w.nT + 1;
   w.tinv = w.logdet + 1;
-  w.work = w.tinv + 4096;
+  w.work = base + work_offset(n, w.nT);
   w.work_doubles = work;
   w.flags = u;
   w.epoch = u + nflags;
   w.info = u + nflags + 1;
   w.err = reinterpret_cast<int*>(u + nflags + 2);
+  w.sweep_count = reinterpret_cast<int*>(u + nflags + 6);
+  w.wait_ticks = bta::flow_spin_ticks(device, 20.0);
+  if (hipDeviceGetAttribute(&w.cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || w.cus < 1)
+    w.cus = 1;
   w.base_bytes = nd * sizeof(double) + (nflags + 2) * sizeof(unsigned long long) + 64;
   int rc = 0;
   if (bta::flow_wanted(w, b)) rc = bta::flow_alloc(w);
@@ -263,10 +272,10 @@ int bta_potrs(bta_ws_t ws, double* D, double* L, double* B, double* T, int n, in
   hipStream_t st = as_stream(stream);
   rc = ensure_inverses(ws, D, n, b, st);
   if (rc) return rc;
-  // the sweeps are a few GEMV launches per block: launched directly (a graph
-  // per right-hand-side buffer would grow without bound)
+  // a sweep is a few launches: made directly (a graph per right-hand-side
+  // buffer would grow without bound)
   std::lock_guard<std::mutex> g(ws->mu);
-  return bta::potrs_enqueue(ws->w, D, L, B, T, n, b, a, rhs, nrhs, ldrhs, trans, st);
+  return bta::potrs_enqueue(ws->w, L, B, n, b, a, rhs, nrhs, ldrhs, trans, st);
 }
 
 int bta_logdet(bta_ws_t ws, const double* D, const double* T, int n, int b, int a, double* out, void* stream) {

@@ -113,27 +113,6 @@ inline GemmJob& add_seg(GemmJob& j, const GemmSeg& s) {
   return j;
 }
 
-// y = beta*y + sum_s alpha_s * op(A_s) x_s, with x and y row-major k x nrhs /
-// m x nrhs blocks (leading dimensions ldx / ldy: one column per right-hand side).
-struct GemvSeg {
-  const double* A;
-  const double* x;
-  double alpha;
-  int k;      // length of x (columns of op(A))
-  int lda, ldx;
-  int ta;     // 0: A (m x k), 1: A^T (A is k x m)
-  int tri;    // 1: op(A) lower (k <= i), 2: op(A) upper (k >= i)
-};
-
-struct GemvJob {
-  double* y;
-  double beta;
-  int m, ldy, nrhs;
-  int nseg;
-  GemvSeg seg[3];
-};
-
-
 // A set of grouped-GEMM launches whose job tables live in device memory.  Built
 // once (hipMalloc + hipMemcpy, never during stream capture), then launched any
 // number of times, including from inside a captured hipGraph.
@@ -158,10 +137,5 @@ struct DevPlan {
   void launch(int idx, hipStream_t st, int variant = 0) const;
   bool empty() const { return launches.empty(); }
 };
-
-// form_t = 1 (op(A) = A^T) needs gemv_scratch(g, 1) doubles of scratch; y may
-// then alias an x of the job (the partial sums are complete before y is written).
-size_t gemv_scratch(const GemvJob& g, int form_t);
-void gemv_launch(const GemvJob& g, int form_t, double* scratch, hipStream_t st);
 
 }  // namespace bta

@@ -1,4 +1,4 @@
-// Grouped FP64 GEMM and GEMV kernels + device job-table plans.
+// Grouped FP64 GEMM kernels + device job-table plans.
 #include <algorithm>
 #include <stdexcept>
 
@@ -724,151 +724,6 @@ __global__ void __launch_bounds__(BTA_THREADS, 1) k_gemm_grouped_big(const GemmJ
       }
 }
 
-// ------------------------------------------------------------------- GEMV
-//
-// Memory-bound sweeps: every matrix element is read once, so the kernels are
-// shaped for bandwidth.  N form (op(A) = A): one wave per output row; with a
-// single unit-stride right-hand side each lane reads two consecutive doubles
-// per access, four accesses in flight, and a butterfly combines the lanes.
-// T form (op(A) = A^T): two passes.  Workgroup (64-column block, K chunk of
-// 128 rows) sums its rows for 64 columns (one per lane, the four waves take
-// every fourth row, four rows in flight) into a partial vector; a second
-// kernel adds the partials of each column in chunk order into y.  Both
-// orders of summation are fixed, so results are reproducible run to run.
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-#define GEMV_TK 128  // rows of A per T-form chunk
-
-__global__ void __launch_bounds__(BTA_THREADS) k_gemv_n(GemvJob g) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int i = blockIdx.x * 4 + w;
-  if (i >= g.m) return;
-  for (int c = 0; c < g.nrhs; ++c) {
-    double acc = 0.0;
-    for (int s = 0; s < g.nseg; ++s) {
-      const GemvSeg& sg = g.seg[s];
-      int kmin = 0, kmax = sg.k;
-      if (sg.tri == 1) kmax = min(kmax, i + 1);
-      if (sg.tri == 2) kmin = i;
-      const double* a = sg.A + (int64_t)i * sg.lda;
-      double p[4] = {0.0, 0.0, 0.0, 0.0};
-      const bool vec = sg.ldx == 1 && g.nrhs == 1 && (sg.lda & 1) == 0 &&
-                       ((reinterpret_cast<uintptr_t>(sg.A) | reinterpret_cast<uintptr_t>(sg.x)) & 15) == 0;
-      if (vec) {
-        // pairs [k0, ke2) as double2; all 16 loads of a 2048-wide stretch are
-        // issued before the first FMA (addresses clamped into the row, the
-        // FMAs masked), so a row of up to 2048 costs one memory round trip
-        const int k0 = kmin & ~1, ke2 = kmax & ~1;
-        for (int base = k0; base < ke2; base += 2048) {
-          double2 av[16], xv[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int kk = min(base + 128 * u + 2 * lane, ke2 - 2);
-            av[u] = *reinterpret_cast<const double2*>(a + kk);
-            xv[u] = *reinterpret_cast<const double2*>(sg.x + kk);
-          }
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int kk = base + 128 * u + 2 * lane;
-            if (kk < ke2) {
-              const double t = fma(av[u].y, xv[u].y, p[u & 3]);
-              p[u & 3] = (kk >= kmin) ? fma(av[u].x, xv[u].x, t) : t;
-            }
-          }
-        }
-        if ((kmax & 1) && kmax - 1 >= kmin && lane == 0) p[0] = fma(a[kmax - 1], sg.x[kmax - 1], p[0]);
-      } else {
-        for (int base = kmin; base < kmax; base += 256) {
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int kk = base + 64 * u + lane;
-            if (kk < kmax) p[u] = fma(a[kk], sg.x[(int64_t)kk * sg.ldx + c], p[u]);
-          }
-        }
-      }
-      acc = fma(sg.alpha, wave_sum((p[0] + p[1]) + (p[2] + p[3])), acc);
-    }
-    if (lane == 0) {
-      double* yp = g.y + (int64_t)i * g.ldy + c;
-      *yp = (g.beta != 0.0) ? fma(g.beta, *yp, acc) : acc;
-    }
-  }
-}
-
-__host__ __device__ inline int gemv_t_chunks(const GemvJob& g) {
-  int n = 0;
-  for (int s = 0; s < g.nseg; ++s) n += (g.seg[s].k + GEMV_TK - 1) / GEMV_TK;
-  return n;
-}
-
-// part[(q * m + j) * nrhs + rc]: alpha_s * sum over chunk q's rows of A[k][j] x[k].
-__global__ void __launch_bounds__(BTA_THREADS) k_gemv_t_part(GemvJob g, double* __restrict__ part) {
-  __shared__ double red[4][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int j = blockIdx.x * 64 + lane;
-  int q = blockIdx.y, s = 0;
-  while (s < g.nseg - 1) {
-    const int nc = (g.seg[s].k + GEMV_TK - 1) / GEMV_TK;
-    if (q < nc) break;
-    q -= nc;
-    ++s;
-  }
-  const GemvSeg& sg = g.seg[s];
-  const int kb = q * GEMV_TK, ke = min(sg.k, kb + GEMV_TK);
-  int klo = kb, khi = ke;  // this lane's rows (triangular operands)
-  if (sg.tri == 1) khi = min(khi, j + 1);
-  if (sg.tri == 2) klo = max(klo, j);
-  const bool col = j < g.m;
-  const int jc = min(j, g.m - 1);
-  const int wu = __builtin_amdgcn_readfirstlane(w);
-  // a chunk outside the triangle for every column of this workgroup loads nothing
-  const int j0 = blockIdx.x * 64, j1 = min(j0 + 64, g.m) - 1;
-  const int nh = ((sg.tri == 1 && kb > j1) || (sg.tri == 2 && ke - 1 < j0)) ? 0 : GEMV_TK / 64;
-  for (int rc = 0; rc < g.nrhs; ++rc) {
-    double p[4] = {0.0, 0.0, 0.0, 0.0};
-    // wave w takes rows kb + w + 4r (r < 32) in two batches of 16 whose loads
-    // are all issued before their FMAs (addresses clamped into the chunk,
-    // the FMAs masked)
-#pragma unroll 1
-    for (int h = 0; h < nh; ++h) {
-      double av[16], xv[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kc = min(kb + wu + 4 * (16 * h + r), ke - 1);  // uniform: x from scalar loads
-        av[r] = sg.A[(int64_t)kc * sg.lda + jc];
-        xv[r] = sg.x[(int64_t)kc * sg.ldx + rc];
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int k = kb + w + 4 * (16 * h + r);
-        if (col && k < ke && k >= klo && k < khi) p[r & 3] = fma(av[r], xv[r], p[r & 3]);
-      }
-    }
-    red[w][lane] = (p[0] + p[1]) + (p[2] + p[3]);
-    __syncthreads();
-    if (w == 0 && col)
-      part[((int64_t)blockIdx.y * g.m + j) * g.nrhs + rc] =
-          sg.alpha * ((red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]));
-    __syncthreads();
-  }
-}
-
-__global__ void __launch_bounds__(BTA_THREADS) k_gemv_t_reduce(GemvJob g, const double* __restrict__ part,
-                                                              int nchunk) {
-  const int64_t e = (int64_t)blockIdx.x * BTA_THREADS + threadIdx.x;
-  if (e >= (int64_t)g.m * g.nrhs) return;
-  const int j = (int)(e / g.nrhs), rc = (int)(e % g.nrhs);
-  double acc = 0.0;
-  for (int q = 0; q < nchunk; ++q) acc += part[((int64_t)q * g.m + j) * g.nrhs + rc];
-  double* yp = g.y + (int64_t)j * g.ldy + rc;
-  *yp = (g.beta != 0.0) ? fma(g.beta, *yp, acc) : acc;
-}
-
 // ------------------------------------------------------------------- plans
 
 DevPlan::~DevPlan() { release(); }
@@ -962,23 +817,6 @@ void DevPlan::launch(int idx, hipStream_t st, int variant) const {
   else
     hipLaunchKernelGGL(k_gemm_grouped, dim3(e.tiles), dim3(BTA_THREADS), 0, st, d_jobs + e.job_off,
                        d_prefix + e.pre_off, e.njobs);
-}
-
-size_t gemv_scratch(const GemvJob& g, int form_t) {
-  return form_t ? (size_t)gemv_t_chunks(g) * g.m * g.nrhs : 0;
-}
-
-void gemv_launch(const GemvJob& g, int form_t, double* scratch, hipStream_t st) {
-  if (g.m <= 0) return;
-  if (!form_t) {
-    hipLaunchKernelGGL(k_gemv_n, dim3((g.m + 3) / 4), dim3(BTA_THREADS), 0, st, g);
-    return;
-  }
-  const int nchunk = gemv_t_chunks(g);
-  hipLaunchKernelGGL(k_gemv_t_part, dim3((g.m + 63) / 64, nchunk), dim3(BTA_THREADS), 0, st, g, scratch);
-  const int64_t tot = (int64_t)g.m * g.nrhs;
-  hipLaunchKernelGGL(k_gemv_t_reduce, dim3((unsigned)((tot + BTA_THREADS - 1) / BTA_THREADS)), dim3(BTA_THREADS), 0,
-                     st, g, scratch, nchunk);
 }
 
 }  // namespace bta

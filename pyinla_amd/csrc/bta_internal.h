@@ -21,7 +21,7 @@ enum KernelClass : int {
   KC_PANEL = 0,     // k_panel_step (tile-column factorization)
   KC_UPDATE = 1,    // k_gemm_nt_sub (block updates D_{i+1}, B_{i+1}, T)
   KC_GROUPED = 2,   // k_gemm_grouped (block inverses, selected inversion)
-  KC_GEMV = 3,      // GEMV kernels (triangular sweeps)
+  KC_GEMV = 3,      // triangular sweeps
   KC_BLAS = 4,      // rocBLAS dgemm of the selected inversion (Sigma_{i+1,i} products)
   KC_COUNT = 5
 };
@@ -129,10 +129,13 @@ struct Workspace {
   unsigned long long* info = nullptr;   // first failing pivot (global row), kInfoNone if none
   int* err = nullptr;                   // nonzero: a bounded wait timed out
   double* logdet = nullptr;             // last log-determinant
-  double* work = nullptr;               // scratch for solve / selected inversion
+  double* work = nullptr;               // scratch of the triangular sweeps (128-byte aligned)
   size_t work_doubles = 0;
   double* tinv = nullptr;               // 64 x 64: inverse of the tip factor
   unsigned long long spin_limit = 1ull << 24;
+  int* sweep_count = nullptr;           // arrow partial sums counted (zero between launches)
+  unsigned long long wait_ticks = 0;    // bound on one in-kernel wait of a sweep, s_memrealtime ticks
+  int cus = 1;                          // compute units of the device
   size_t base_bytes = 0;                // bytes of the buffers above
   // Full inverses W_i = D_i^-1 of the diagonal factor blocks (n * b * b),
   // reserved with WS_SOLVE or WS_SELINV.
@@ -277,8 +280,10 @@ int trtri_enqueue(Workspace& ws, const double* D, int n, int b, hipStream_t st);
 int potri_prepare(Workspace& ws, double* D, double* L, double* B, double* T, int n, int b, int a);
 int potri_enqueue(Workspace& ws, double* D, double* L, double* B, double* T, int n, int b, int a,
                   hipStream_t st);
-int potrs_enqueue(Workspace& ws, const double* D, const double* L, const double* B, const double* T,
-                  int n, int b, int a, double* rhs, int nrhs, int ldrhs, int trans, hipStream_t st);
+int potrs_enqueue(Workspace& ws, const double* L, const double* B, int n, int b, int a, double* rhs, int nrhs,
+                  int ldrhs, int trans, hipStream_t st);
+// Doubles of the scratch the sweeps hand their vectors over in.
+size_t sweep_doubles(int n, int b);
 // 2 sum log diag(D_i) (+ 2 sum log diag(T) if a > 0) of the blocks as they are
 // held, in a fixed summation order, written to out (device).
 int logdet_enqueue(const double* D, const double* T, int n, int b, int a, double* part, double* out,
