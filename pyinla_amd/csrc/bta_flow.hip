@@ -465,10 +465,10 @@ __device__ __forceinline__ int flow_poll(const FlowArgs& p, unsigned long long* 
 // workgroup has in flight (the prefetched accumulator of the step).
 __device__ __forceinline__ bool flow_wait2(const FlowArgs& p, unsigned long long* f1, unsigned long long* f2,
                                            unsigned long long tag, int* ok_sh) {
-  if (threadIdx.x == 0) {
-    int ok = flow_poll(p, f1, tag);
-    if (ok) ok = flow_poll(p, f2, tag);
-    *ok_sh = ok;
+  if (threadIdx.x < 64) {  // lanes 0 and 1 poll one flag each, side by side
+    const int ok = threadIdx.x < 2 ? flow_poll(p, threadIdx.x == 0 ? f1 : f2, tag) : 1;
+    const bool all = __ballot(ok == 0) == 0;
+    if (threadIdx.x == 0) *ok_sh = all ? 1 : 0;
   }
   lds_barrier();
   const int ok = *ok_sh;
@@ -476,23 +476,62 @@ __device__ __forceinline__ bool flow_wait2(const FlowArgs& p, unsigned long long
   return ok != 0;
 }
 
-// 64x64 contiguous tile <-> registers / LDS with system-scope accesses.
-__device__ __forceinline__ void lds_load_sys(double* __restrict__ s, const double* __restrict__ g) {
-  const int c = threadIdx.x & 63;
-#pragma unroll 4
-  for (int r = threadIdx.x >> 6; r < 64; r += 4) s[r * BTA_LDS_LD + c] = ld_sys(&g[r * 64 + c]);
-}
-
 // Stores, after the caller's st_sys data stores, the flag once they completed.
 __device__ __forceinline__ void flow_publish(unsigned long long* flag, unsigned long long tag) {
   flag_publish(flag, tag);
 }
 
-// X = C inv(L_kk)^T from C in sC and inv(L_kk) (lower) in sW.
-__device__ __forceinline__ void flow_trsm(TileAcc& x, const double* sC, const double* sW) {
-  acc_zero(x);
-  const int kend = ((threadIdx.x >> 6) & 1) * 32 + 32;
-  mma_nt<false>(x, sC, sW, 0, kend);
+// X = C inv(L_kk)^T, rows 16w .. 16w+15 by wave w: C in sC, inv(L_kk) (lower) in
+// sW.  Element q of x.c[cb / 2][cb % 2] is row 16w + 4q + lane / 16, column
+// 16cb + lane % 16.  The
+// triangular inverse leaves 10 of 16 block products: 40 MFMAs for every wave
+// (split in 32 x 32 quadrants, two of the waves have 64).
+__device__ __forceinline__ void tile_solve(TileAcc& x, const double* sC, const double* sW) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  double a[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) a[t] = sC[(16 * w + li) * BTA_LDS_LD + 4 * t + lk];
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) x.c[cb >> 1][cb & 1] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int cb = m; cb < 4; ++cb)
+        x.c[cb >> 1][cb & 1] = mfma_f64(a[4 * m + t], sW[(16 * cb + li) * BTA_LDS_LD + 16 * m + 4 * t + lk],
+                                        x.c[cb >> 1][cb & 1]);
+    __builtin_amdgcn_sched_barrier(0);  // bounds the operands read ahead (registers)
+  }
+}
+
+// Stores of tile_solve's result: factor tile (rows x cols of it, row stride ld)
+// and exchange tile.
+__device__ __forceinline__ void solve_store(const TileAcc& x, double* g, int64_t ld, int rows, int cols) {
+  const int lane = threadIdx.x & 63;
+  const int i0 = 16 * (threadIdx.x >> 6) + (lane >> 4), j0 = lane & 15;
+  gdouble* t = gview(g) + (int64_t)i0 * ld + j0;
+  if (rows == 64 && cols == 64) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) t[4 * q * ld + 16 * cb] = x.c[cb >> 1][cb & 1][q];
+  } else {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (i0 + 4 * q < rows && j0 + 16 * cb < cols) t[4 * q * ld + 16 * cb] = x.c[cb >> 1][cb & 1][q];
+  }
+}
+__device__ __forceinline__ void solve_store_sys(const TileAcc& x, double* g) {
+  const int lane = threadIdx.x & 63;
+  double* t = g + (16 * (threadIdx.x >> 6) + (lane >> 4)) * 64 + (lane & 15);
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) st_sys(t + 4 * q * 64 + 16 * cb, x.c[cb >> 1][cb & 1][q]);
 }
 
 // Chain: store the factored diagonal tile k held in sA (L_kk) / sB (inverse).
@@ -511,77 +550,228 @@ __device__ __forceinline__ void chain_store_inv(const FlowArgs& p, int k, const 
   }
 }
 
-// ... then, after the inverse's flag, L_kk to the factor (read by no helper)
-// and the tile's log pivots.
-__device__ __forceinline__ void chain_store_l(const FlowArgs& p, int k, const TileCholResult& res,
-                                              const double* sA) {
+// ... then, after the inverse's flag, L_kk to the factor (no helper reads it;
+// the strict upper triangle as zeros, whatever sA holds there).
+__device__ __forceinline__ void chain_store_l(const FlowArgs& p, int k, const double* sA) {
   int rows, cols;
   double* g = flow_tile(p, k, k, rows, cols);
   const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
-  for (int r = r0; r < 64; r += 4)
-    if (r < rows && c < cols) g[(int64_t)r * p.b + c] = sA[r * BTA_LDS_LD + c];
-  if (threadIdx.x == 0) {
+  gdouble* t = gview(g) + (int64_t)r0 * p.b + c;
+#pragma unroll
+  for (int h = 0; h < 16; h += 8) {
+    double v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = r0 + 4 * (h + j);
+      const double x = sA[r * BTA_LDS_LD + c];
+      v[j] = c <= r ? x : 0.0;
+    }
+    if (rows == 64) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[(int64_t)4 * (h + j) * p.b] = v[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (r0 + 4 * (h + j) < rows && c < cols) t[(int64_t)4 * (h + j) * p.b] = v[j];
+    }
+  }
+}
+
+// The log pivots of tile k from its diagonal (lane i: l_ii), by one wave.
+__device__ __forceinline__ void chain_log(const FlowArgs& p, int k, double lii) {
+  const TileCholResult res = tile_log_pivots(lii, min(64, p.b - 64 * k));
+  if ((threadIdx.x & 63) == 0) {
     p.logpart[k] = res.logsum;
     if (res.fail >= 0) atomicMin(p.info, (unsigned long long)(p.row0 + (long long)k * 64 + res.fail));
   }
 }
 
+// Current value of a flag (`tag` for an absent flag).
+__device__ __forceinline__ unsigned long long flag_value(const unsigned long long* f, unsigned long long tag) {
+  return f == nullptr ? tag
+                      : __hip_atomic_load(const_cast<unsigned long long*>(f), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// 16x16 block (bi, bj), bi >= bj, of the lower triangle of a rows x rows
+// row-major tile (0 outside it) in the accumulator layout; a diagonal block is
+// mirrored.  (Clamped addresses and selects: loads under tests are waited for
+// one by one.)
+__device__ __forceinline__ f64x4 block_load(const double* __restrict__ g, int ld, int rows, int bi, int bj, int lane) {
+  f64x4 v;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int i0 = 16 * bi + 4 * q + (lane >> 4), j0 = 16 * bj + (lane & 15);
+    const int i = max(i0, j0), j = min(i0, j0);
+    const double x = gview(g)[(unsigned)(min(i, rows - 1) * ld + min(j, rows - 1))];
+    v[q] = i < rows ? x : 0.0;
+  }
+  return v;
+}
+
 // Per column k the chain
 //   1. waits for the hand-off tiles (k+1, k) and (k+1, k+1) (updated by their
-//      helpers through column k-1) and loads both;
-//   2. solves X = C(k+1, k) inv(L_kk)^T and issues the stores of X;
-//   3. applies C(k+1, k+1) -= X X^T, then publishes X (its stores drained
-//      during the update);
-//   4. factors C(k+1, k+1), stores its inverse and publishes it at once (the
-//      helpers' solves of column k+1 wait for it; the stores drain while
-//      they are issued, a few hundred cycles of wait measured on MI355X),
-//      then stores L into the factor (no helper reads it; those stores drain
-//      during the next step's wait).
-__device__ void flow_chain(const FlowArgs& p, unsigned long long tag, double* sA, double* sB,
+//      helpers through column k-1), issues the loads of both and meanwhile
+//      stores L_kk into the factor;
+//   2. solves X = C(k+1, k) inv(L_kk)^T, 16 rows per wave, so that a wave's rows
+//      of C and X are its own and nothing waits for another wave until X is
+//      complete;
+//   3. applies C(k+1, k+1) -= X X^T, lower 16x16 blocks only: wave 0 takes the
+//      first block and factors it at once; the others take three blocks each,
+//      store X and publish it (the helpers' updates of the next hand-off tile
+//      wait for it);
+//   4. factors the rest of C(k+1, k+1), stores its inverse and publishes it at
+//      once (the helpers' solves of column k+1 wait for it).  The log pivots of
+//      tile k are taken by wave 3 beside the last 16x16 factorization.
+// Measured on MI355X at b = 417, us per column: 15.2, against 20.7 with both
+// products as 32 x 32 quadrants one after the other, X published behind them, L
+// stored and the logarithms taken before the next wait, and the 16x16 blocks
+// factored by column.
+__device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long tag, double* sA, double* sB,
                            int* ok_sh) {
   const int nT = p.nT;
-  int rows, cols;
-  TileAcc acc, accd;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lk = lane >> 4;
   {
+    int rows, cols;
     const double* g = flow_tile(p, 0, 0, rows, cols);
+    TileAcc acc;
     acc_load(acc, g, p.b, rows, cols);
     acc_to_lds(acc, sA);
     __syncthreads();
-    const TileCholResult res = tile_chol_inv(sA, sB, rows);
+    tile_chol_inv(sA, sB, rows);
     chain_store_inv(p, 0, sB);
     flow_publish(wflag(p, 0), tag);
-    chain_store_l(p, 0, res, sA);
   }
+  // blocks of the diagonal tile that wave w updates (wave 0: only the first)
+  const int bi0 = w, bj0 = 0;
+  const int bi1 = max(w, 1), bj1 = 1;
+  const int bi2 = w == 1 ? 3 : max(w, 2), bj2 = w == 1 ? 3 : 2;
+  bool ready = true;  // the hand-off flags of this column were seen set
   for (int k = 0; k + 1 < nT; ++k) {
-    if (k == 0) {
-      acc_load(acc, flow_tile(p, 1, 0, rows, cols), p.b, rows, cols);
-      acc_load(accd, flow_tile(p, 1, 1, rows, cols), p.b, rows, cols);
-    } else {
-      if (!flow_wait2(p, hflag(p, k, 0), hflag(p, k, 1), tag, ok_sh) && threadIdx.x == 0) atomicOr(p.err, 2);
-      acc_load_sys(acc, hsub(p, k));
-      acc_load_sys(accd, hdiag(p, k + 1));
+    const int mv = min(64, p.b - 64 * (k + 1));
+    int rows, cols;
+    double* gx = flow_tile(p, k + 1, k, rows, cols);
+    const double* gc = gx;
+    const double* gd = flow_tile(p, k + 1, k + 1, rows, cols);
+    int ld = p.b;
+    rows = mv;
+    // opaque, so that the addresses below are formed here and not kept (spilled)
+    // across the columns
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    if (k > 0) {
+      if (!ready && !flow_wait2(p, hflag(p, k, 0), hflag(p, k, 1), tag, ok_sh) && threadIdx.x == 0) atomicOr(p.err, 2);
+      // final values, read by nobody on this XCD before: ordinary loads
+      gc = hsub(p, k);
+      gd = hdiag(p, k + 1);
+      ld = 64;
     }
-    acc_to_lds(acc, sA);
-    __syncthreads();
-    flow_trsm(acc, sA, sB);  // X(k+1, k) in acc
-    lds_barrier();           // the reads of sA are done
-    {
-      double* g = flow_tile(p, k + 1, k, rows, cols);
-      acc_store(acc, g, p.b, rows, cols);
-      acc_store_sys(acc, xtile(p, k + 1, k));
-      acc_to_lds(acc, sA);
+    // C rows 16w .. 16w+15 as pairs: row 2q + lane / 32, columns 2 (lane % 32), +1
+    double c[16];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const unsigned at = min(16 * w + 2 * q + (ln >> 5), rows - 1) * ld + 2 * (ln & 31);
+      c[2 * q] = gview(gc)[at];
+      c[2 * q + 1] = gview(gc)[at + 1];
+    }
+    f64x4 d0 = block_load(gd, ld, rows, bi0, bj0, ln);
+    f64x4 d1 = block_load(gd, ld, rows, bi1, bj1, ln);
+    f64x4 d2 = block_load(gd, ld, rows, bi2, bj2, ln);
+    // while those loads are in flight: L_kk out of sA
+    chain_store_l(p, k, sA);
+    const double lii = sA[lane * BTA_LDS_LD + lane];
+    if (threadIdx.x == 0) ok_sh[1] = 0;  // waves whose stores of X have completed
+    lds_barrier();
+    // the wave's rows of C through its own rows of sA into MFMA operands
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int r = 16 * w + 2 * q + (lane >> 5);
+      const bool in = r < rows;
+      *(f64x2*)&sA[r * BTA_LDS_LD + 2 * (lane & 31)] = f64x2{in ? c[2 * q] : 0.0, in ? c[2 * q + 1] : 0.0};
+    }
+    TileAcc x;
+    tile_solve(x, sA, sB);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sA[(16 * w + 4 * q + lk) * BTA_LDS_LD + 16 * cb + li] = x.c[cb >> 1][cb & 1][q];
+    lds_barrier();  // X is complete in sA
+    f64x4 e0;
+    if (w == 0) {
+      f64x4 d0b = f64x4{0.0, 0.0, 0.0, 0.0};  // two chains of dependent MFMAs
+#pragma unroll
+      for (int t = 0; t < 16; t += 2) {
+        const double u = sA[li * BTA_LDS_LD + 4 * t + lk], v = sA[li * BTA_LDS_LD + 4 * t + 4 + lk];
+        d0 = mfma_f64_nega(u, u, d0);
+        d0b = mfma_f64_nega(v, v, d0b);
+      }
+      d0 += d0b;
+      if (mv == 64) chol16_inv16(d0, e0);
+    } else {
+      // X to the exchange tile: the wave's rows, and a third of wave 0's
+      double* xt = xtile(p, k + 1, k);
+      solve_store_sys(x, xt);
+#pragma unroll
+      for (int h = 0; h < 6; ++h) {
+        const int r = min(w - 1 + 3 * h, 15);
+        st_sys(xt + r * 64 + ln, sA[r * BTA_LDS_LD + ln]);
+      }
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const double a0 = sA[(16 * bi0 + li) * BTA_LDS_LD + 4 * t + lk];
+        const double a2 = sA[(16 * bi2 + li) * BTA_LDS_LD + 4 * t + lk];
+        const double b0 = sA[(16 * bj0 + li) * BTA_LDS_LD + 4 * t + lk];
+        const double b1 = sA[(16 * bj1 + li) * BTA_LDS_LD + 4 * t + lk];
+        const double b2 = sA[(16 * bj2 + li) * BTA_LDS_LD + 4 * t + lk];
+        d0 = mfma_f64_nega(a0, b0, d0);
+        d1 = mfma_f64_nega(a0, b1, d1);
+        d2 = mfma_f64_nega(a2, b2, d2);
+        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      // the last of the three waves whose stores have completed publishes X
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      if (lane == 0 && atomicAdd(&ok_sh[1], 1) == 2)
+        __hip_atomic_store(xflag(p, k + 1, k), tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      // ... and to the factor
+      solve_store(x, gx, p.b, rows, 64);
+#pragma unroll
+      for (int h = 0; h < 6; ++h) {
+        const int r = min(w - 1 + 3 * h, min(15, rows - 1));
+        gview(gx)[(unsigned)(r * p.b + ln)] = sA[r * BTA_LDS_LD + ln];
+      }
+    }
+    lds_barrier();  // X in sA and inv(L_kk) in sB are no longer read
+    if (w == 0) {
+      if (mv == 64) store_chol16(d0, e0, sA, sB, 0);
+      else store16(sA, 0, 0, d0);
+    } else {
+      store16(sA, 16 * bi0, 16 * bj0, d0);
+      store16(sA, 16 * bi1, 16 * bj1, d1);
+      store16(sA, 16 * bi2, 16 * bj2, d2);
     }
     lds_barrier();
-    mma_nt64<true>(accd, sA, sA);
-    flow_publish(xflag(p, k + 1, k), tag);
-    acc_to_lds(accd, sA);
-    __syncthreads();
-    const int mv = min(64, p.b - 64 * (k + 1));
-    const TileCholResult res = tile_chol_inv(sA, sB, mv);
+    if (mv == 64) {
+      tile_chol_blocks<true>(sA, sB, 64, [&] { chain_log(p, k, lii); });
+    } else {
+      tile_chol_inv(sA, sB, mv);
+      if (w == 3) chain_log(p, k, lii);
+    }
     chain_store_inv(p, k + 1, sB);
+    // the hand-off flags of the next column, loaded while the stores drain
+    unsigned long long hv = tag;
+    if (k + 2 < nT && threadIdx.x < 2) hv = flag_value(hflag(p, k + 1, threadIdx.x), tag);
+    if (threadIdx.x < 64) {
+      const bool all = __ballot(hv != tag) == 0;
+      if (threadIdx.x == 0) ok_sh[0] = all ? 1 : 0;
+    }
     flow_publish(wflag(p, k + 1), tag);
-    chain_store_l(p, k + 1, res, sA);
+    ready = ok_sh[0] != 0;
   }
+  chain_store_l(p, nT - 1, sA);
+  if (w == 0) chain_log(p, nT - 1, sA[lane * BTA_LDS_LD + lane]);
 }
 
 // One step of a helper: a task, or one column kk of a next-block task.
@@ -628,13 +818,6 @@ __device__ __forceinline__ HStep make_step(const FlowArgs& p, int t, int kk) {
   return st;
 }
 
-// Current value of a flag (`tag` for an absent flag).
-__device__ __forceinline__ unsigned long long flag_value(const unsigned long long* f, unsigned long long tag) {
-  return f == nullptr ? tag
-                      : __hip_atomic_load(const_cast<unsigned long long*>(f), __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // Issue the operand loads of a step into registers.  The exchange tiles and
 // tile inverses are written once per launch (before their flag), so ordinary
 // cached loads after the flag see them; the L2 lines cannot be older than the
@@ -644,7 +827,7 @@ __device__ __forceinline__ void step_fetch(const HStep& st, TilePrefetch& pa, Ti
   if (st.srcB && st.srcB != st.srcA) pb.load_full(st.srcB);
 }
 
-__device__ void flow_helper(const FlowArgs& p, int h, unsigned long long tag, double* sA, double* sB,
+__device__ __forceinline__ void flow_helper(const FlowArgs& p, int h, unsigned long long tag, double* sA, double* sB,
                             int* ok_sh) {
   const int nT = p.nT;
   const int t0 = p.off[h], t1 = p.off[h + 1];
@@ -734,10 +917,10 @@ __device__ void flow_helper(const FlowArgs& p, int h, unsigned long long tag, do
     if (fetched && !pf_mma) step_fetch(nxt, pa, pb);
     const double* sBop = (cur.srcB == cur.srcA) ? sA : sB;
     if (cur.op == FLOW_TRSM) {
-      flow_trsm(acc, sA, sB);  // the accumulator was staged in sA: reuse its registers
+      tile_solve(acc, sA, sB);  // the accumulator was staged in sA: reuse its registers
       lds_barrier();
-      acc_store(acc, g, p.b, rows, cols);
-      acc_store_sys(acc, xtile(p, cur.rho, cur.c));
+      solve_store(acc, g, p.b, rows, cols);
+      solve_store_sys(acc, xtile(p, cur.rho, cur.c));
       carry_rho = carry_c = -1;
       flow_publish(xflag(p, cur.rho, cur.c), tag);
     } else {

@@ -147,7 +147,8 @@ __device__ __forceinline__ void panel_body(const PanelArgs& p, int idx, double* 
     acc_to_lds(acc, sA);
     __syncthreads();
     const int mv = rows;  // == cols
-    const TileCholResult res = tile_chol_inv(sA, sB, mv);
+    tile_chol_inv(sA, sB, mv);
+    const TileCholResult res = tile_chol_result(sA, mv);
     // store L_kk (full tile: zero strict upper) and inv(L_kk)
     {
       const int c = threadIdx.x & 63;
@@ -328,7 +329,8 @@ __global__ void __launch_bounds__(BTA_THREADS) k_tip_potrf(double* T, int a, dou
   __shared__ double sB[64 * BTA_LDS_LD];
   lds_load_tile(sA, T, a, a, a);
   __syncthreads();
-  const TileCholResult res = tile_chol_inv(sA, sB, a);
+  tile_chol_inv(sA, sB, a);
+  const TileCholResult res = tile_chol_result(sA, a);
   const int c = threadIdx.x & 63;
   for (int r = threadIdx.x >> 6; r < 64; r += 4) {
     if (r < a && c < a) T[(int64_t)r * a + c] = sA[r * BTA_LDS_LD + c];
@@ -365,7 +367,8 @@ __global__ void __launch_bounds__(BTA_THREADS) k_tip_potrf_batched(const ProbDes
   if (a <= 0) return;
   lds_load_tile(sA, d.T, a, a, a);
   __syncthreads();
-  const TileCholResult res = tile_chol_inv(sA, sB, a);
+  tile_chol_inv(sA, sB, a);
+  const TileCholResult res = tile_chol_result(sA, a);
   const int c = threadIdx.x & 63;
   for (int r = threadIdx.x >> 6; r < 64; r += 4) {
     if (r < a && c < a) d.T[(int64_t)r * a + c] = sA[r * BTA_LDS_LD + c];
