@@ -142,27 +142,6 @@ struct TilePrefetch {
       for (int j = 0; j < 16; ++j) s[c * BTA_LDS_LD + r0 + 4 * j] = r[j];
     }
   }
-  // A full, contiguous 64 x 64 tile (ld 64) as 128-bit pairs: pair q of the
-  // thread is columns 2 (t % 32), +1 of row t / 32 + 8 q (one wave: two whole
-  // rows per load), half the load and LDS-store instructions of load/store.
-  __device__ __forceinline__ static const gf64x2* full_pair(const double* __restrict__ g, int q) {
-    const int t = threadIdx.x;
-    return (const gf64x2*)(gview(g) + ((t >> 5) + 8 * q) * 64 + 2 * (t & 31));
-  }
-  __device__ __forceinline__ void set_pair(int q, f64x2 v) {
-    r[2 * q] = v.x;
-    r[2 * q + 1] = v.y;
-  }
-  __device__ __forceinline__ void load_full(const double* __restrict__ g) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) set_pair(q, *full_pair(g, q));
-  }
-  __device__ __forceinline__ void store_full(double* __restrict__ s) const {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < 8; ++q)
-      *(f64x2*)&s[((t >> 5) + 8 * q) * BTA_LDS_LD + 2 * (t & 31)] = f64x2{r[2 * q], r[2 * q + 1]};
-  }
 };
 
 // acc += sign * sA(64 x K) * sB(64 x K)^T over k in [0, kmax), kmax % 4 == 0.
@@ -208,8 +187,7 @@ __device__ __forceinline__ void lds_barrier() {
 // fragments of k step t+1 read while the MFMAs of step t run (two fragment
 // register sets; the scheduling barriers keep each step's reads ahead of the
 // previous step's MFMAs, which LLVM otherwise sinks behind them and then
-// waits for).  A helper runs one wave per SIMD, so nothing else hides the
-// LDS latency.
+// waits for): with one or two waves per SIMD nothing else hides the LDS latency.
 template <bool NEG>
 __device__ __forceinline__ void mma_nt64(TileAcc& t, const double* __restrict__ sA,
                                          const double* __restrict__ sB) {
@@ -244,56 +222,6 @@ __device__ __forceinline__ void mma_nt64(TileAcc& t, const double* __restrict__ 
     if (k + 4 < 64) {
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // the 4 LDS reads of step k+4
       __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  // then the 4 MFMAs of step k
-    }
-    a0 = n0;
-    a1 = n1;
-    b0 = m0;
-    b1 = m1;
-  }
-}
-
-// mma_nt64<true> that also loads the next step's two operand tiles (64 x 64,
-// contiguous) into the prefetch registers, one 128-bit load per k step, so
-// that the load issue overlaps the MFMAs instead of preceding them.  Same
-// registers and layout as TilePrefetch::load_full.
-__device__ __forceinline__ void mma_nt64_neg_pf(TileAcc& t, const double* __restrict__ sA,
-                                                const double* __restrict__ sB, double (&ra)[16],
-                                                const double* __restrict__ srcA, double (&rb)[16],
-                                                const double* __restrict__ srcB) {
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-  const int li = lane & 15, lk = lane >> 4;
-  const double* a0p = sA + (wm + li) * BTA_LDS_LD + lk;
-  const double* a1p = sA + (wm + 16 + li) * BTA_LDS_LD + lk;
-  const double* b0p = sB + (wn + li) * BTA_LDS_LD + lk;
-  const double* b1p = sB + (wn + 16 + li) * BTA_LDS_LD + lk;
-  double a0 = a0p[0], a1 = a1p[0], b0 = b0p[0], b1 = b1p[0];
-#pragma unroll
-  for (int k = 0; k < 64; k += 4) {
-    double n0 = 0.0, n1 = 0.0, m0 = 0.0, m1 = 0.0;
-    if (k + 4 < 64) {
-      n0 = a0p[k + 4];
-      n1 = a1p[k + 4];
-      m0 = b0p[k + 4];
-      m1 = b1p[k + 4];
-    }
-    const int j = k >> 2;  // k step: pair j / 2 of operand A (even) or B (odd)
-    const f64x2 v = *TilePrefetch::full_pair((j & 1) ? srcB : srcA, j >> 1);
-    if (j & 1) {
-      rb[j - 1] = v.x;
-      rb[j] = v.y;
-    } else {
-      ra[j] = v.x;
-      ra[j + 1] = v.y;
-    }
-    t.c[0][0] = mfma_f64_nega(a0, b0, t.c[0][0]);
-    t.c[0][1] = mfma_f64_nega(a0, b1, t.c[0][1]);
-    t.c[1][0] = mfma_f64_nega(a1, b0, t.c[1][0]);
-    t.c[1][1] = mfma_f64_nega(a1, b1, t.c[1][1]);
-    if (k + 4 < 64) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads of step k+4
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one prefetch load
-      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  // MFMAs of step k
     }
     a0 = n0;
     a1 = n1;
@@ -382,17 +310,8 @@ __device__ __forceinline__ double ld_sys(const double* p) {
   return __hip_atomic_load(const_cast<double*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// A 64 x 64 accumulator tile to / from a contiguous 64 x 64 buffer with
-// system-scope stores / loads.
-__device__ __forceinline__ void acc_load_sys(TileAcc& t, const double* __restrict__ g) {
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) t.c[x][y][r] = ld_sys(&g[acc_row(x, r) * 64 + acc_col(y)]);
-}
-
+// A 64 x 64 accumulator tile to a contiguous 64 x 64 buffer with system-scope
+// stores.
 __device__ __forceinline__ void acc_store_sys(const TileAcc& t, double* __restrict__ g) {
 #pragma unroll
   for (int x = 0; x < 2; ++x)

@@ -34,11 +34,13 @@
 // Memory protocol (the L2 caches of the XCDs are not coherent): every address
 // is stored to by one workgroup only.  Helpers accumulate their tiles in place
 // with ordinary loads and stores; a finished tile is also written once, with
-// system-scope (write-through) stores, to an exchange buffer that readers load
-// with system-scope loads, and a flag carrying the call tag is stored after
-// the data has completed.  The diagonal and sub-diagonal tiles the chain takes
-// over are accumulated by their helpers in a separate hand-off buffer so that
-// only the chain ever stores to their place in the factor.
+// system-scope (write-through) stores, to an exchange buffer, and a flag carrying
+// the call tag is stored after the data has completed.  Readers poll the flag
+// past the caches and then read the tile, in the order of MFMA operands, with
+// ordinary loads: no cache can hold an older copy from within the launch.  The
+// diagonal and sub-diagonal tiles the chain takes over are accumulated by their
+// helpers in a separate hand-off buffer so that only the chain ever stores to
+// their place in the factor.
 #pragma once
 #include <stdint.h>
 
@@ -108,7 +110,7 @@ struct FlowArgs {
   double* Bn;                // B_{i+1} or nullptr
   double* T;                 // tip (a x a) or nullptr
   double* winv;              // nT tiles: inverse of each diagonal tile of D_i
-  double* xbuf;              // R * nT tiles: exchange copy of every finished tile
+  double* xbuf;              // R * nT tiles: exchange copy of every finished tile, in MFMA operand order
   double* hacc;              // 2 * nT tiles: hand-off accumulators (sub-diagonal, diagonal)
   double* logpart;           // nT partial log sums
   unsigned long long* flags; // R*nT finished tiles, nT tile inverses, 2*nT hand-offs

@@ -143,39 +143,46 @@ static void flow_build_levels(const FlowShape& s, int helpers, int delta, FlowSc
 // launch), so the solves and updates the chain is about to wait for come
 // before bulk updates of tiles needed much later and the next-block updates
 // fill the gaps.  Each helper's list is the order of its tasks in that
-// simulation.  The simulated start times order all tasks, the chain's
-// included, consistently with every dependency and with every list, so with
-// all workgroups resident the earliest unfinished task in that order can
-// always run, whatever the real durations: no interleaving can deadlock.
+// simulation.  The costs and the group size were tuned together on MI355X: with
+// the costs of a slower update (12 k, of which 3 k are saved by a carried
+// accumulator, solve 14.5 k, groups of 2) a lone factorization takes 638 us per
+// block at b = 2000 and a pair 1026; with these 550 and 883 (b = 1600: 379 and
+// 372; b <= 800: the chain's time per column either way).  Solve costs of 12, 16,
+// 20 k: 591, 573, 564 at groups of 8; groups of 4, 8, 12, 16: 609, 584, 567, 599;
+// a margin of 0, 2, 3 instead of 1: 2-4 % slower.
+// The simulated start times order all tasks, the chain's included, consistently
+// with every dependency and with every list, so with all workgroups resident the
+// earliest unfinished task in that order can always run, whatever the real
+// durations: no interleaving can deadlock.
 #ifndef FLOW_COST_CHOL
-#define FLOW_COST_CHOL 30000  // chain: factor + inverse of a diagonal tile, stores, publish
+#define FLOW_COST_CHOL 21000  // chain: factor + inverse of a diagonal tile, stores, publish
 #endif
 #ifndef FLOW_COST_CTRSM
-#define FLOW_COST_CTRSM 10000  // chain: solve of the sub-diagonal tile, stores
+#define FLOW_COST_CTRSM 8000  // chain: solve of the sub-diagonal tile, stores
 #endif
 #ifndef FLOW_COST_CUPD
-#define FLOW_COST_CUPD 4600  // chain: update of the next diagonal tile
+#define FLOW_COST_CUPD 4500  // chain: update of the next diagonal tile
 #endif
 #ifndef FLOW_COST_UPD
-#define FLOW_COST_UPD 12000  // rank-64 update, accumulator loaded and stored
+#define FLOW_COST_UPD 9000  // rank-64 update, accumulator loaded and stored
 #endif
 #ifndef FLOW_COST_CARRY
-#define FLOW_COST_CARRY 3000  // saved when the previous task left the accumulator in registers
+#define FLOW_COST_CARRY 5000  // saved when the previous task left the accumulator in registers
 #endif
 #ifndef FLOW_COST_TRSM
-#define FLOW_COST_TRSM 14500  // tile solve, exchange copy and flag
+#define FLOW_COST_TRSM 24000  // tile solve (11 k), exchange copy, and what a helper behind in its list waits
 #endif
 #ifndef FLOW_COST_NEXTCOL
-#define FLOW_COST_NEXTCOL 10800  // one column of a next-block task
+#define FLOW_COST_NEXTCOL 6000  // one column of a next-block task
 #endif
 #ifndef FLOW_COST_ZERO
 #define FLOW_COST_ZERO 500
 #endif
 #ifndef FLOW_UPD_GROUP
-#define FLOW_UPD_GROUP 2  // columns per held-back update group
+#define FLOW_UPD_GROUP 10  // columns per held-back update group
 #endif
 #ifndef FLOW_UPD_MARGIN
-#define FLOW_UPD_MARGIN 2  // the updates by the last columns before a tile's own are not held back
+#define FLOW_UPD_MARGIN 1  // the updates by the last columns before a tile's own are not held back
 #endif
 #ifndef FLOW_COST_LAT
 #define FLOW_COST_LAT 1500  // flag store to flag seen by another workgroup
@@ -405,7 +412,6 @@ bool flow_build_schedule(const FlowShape& s, int helpers, int delta, FlowSchedul
 
 // ------------------------------------------------------------------ device
 
-
 __device__ __forceinline__ double* flow_tile(const FlowArgs& p, int rho, int c, int& rows, int& cols) {
   cols = min(64, p.b - 64 * c);
   if (rho < p.nT) {
@@ -440,17 +446,19 @@ __device__ __forceinline__ double* hdiag(const FlowArgs& p, int c) {
   return p.hacc + ((int64_t)p.nT + c) * 4096;
 }
 
-// Bounded wait by thread 0 for *flag == tag (nullptr: nothing to wait for).
-// Gives up (returns 0 and raises err) after spin_ticks, or at once when another
-// workgroup has raised err, so that every workgroup still reaches the end of
-// its list.
+// Bounded wait of the calling lane for *flag == tag (nullptr: nothing to wait
+// for).  Gives up (returns 0 and raises err) after spin_ticks, or, after a 1024th
+// of them, when another workgroup has raised err (polled by every wave from the
+// start, that one word would be a hot spot), so that every workgroup still
+// reaches the end of its list.
 __device__ __forceinline__ int flow_poll(const FlowArgs& p, unsigned long long* flag, unsigned long long tag) {
   if (flag == nullptr) return 1;
   if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == tag) return 1;
   const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
   while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != tag) {
-    if (__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0) return 0;
-    if (__builtin_amdgcn_s_memrealtime() - t0 > p.spin_ticks) {
+    const unsigned long long dt = __builtin_amdgcn_s_memrealtime() - t0;
+    if (dt > p.spin_ticks >> 10 && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0) return 0;
+    if (dt > p.spin_ticks) {
       atomicOr(p.err, 1);
       return 0;
     }
@@ -486,8 +494,7 @@ __device__ __forceinline__ void flow_publish(unsigned long long* flag, unsigned 
 // 16cb + lane % 16.  The
 // triangular inverse leaves 10 of 16 block products: 40 MFMAs for every wave
 // (split in 32 x 32 quadrants, two of the waves have 64).
-__device__ __forceinline__ void tile_solve(TileAcc& x, const double* sC, const double* sW) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__device__ __forceinline__ void tile_solve(TileAcc& x, const double* sC, const double* sW, int w, int lane) {
   const int li = lane & 15, lk = lane >> 4;
   double a[16];
 #pragma unroll
@@ -508,9 +515,9 @@ __device__ __forceinline__ void tile_solve(TileAcc& x, const double* sC, const d
 
 // Stores of tile_solve's result: factor tile (rows x cols of it, row stride ld)
 // and exchange tile.
-__device__ __forceinline__ void solve_store(const TileAcc& x, double* g, int64_t ld, int rows, int cols) {
-  const int lane = threadIdx.x & 63;
-  const int i0 = 16 * (threadIdx.x >> 6) + (lane >> 4), j0 = lane & 15;
+__device__ __forceinline__ void solve_store(const TileAcc& x, double* g, int64_t ld, int rows, int cols, int w,
+                                            int lane) {
+  const int i0 = 16 * w + (lane >> 4), j0 = lane & 15;
   gdouble* t = gview(g) + (int64_t)i0 * ld + j0;
   if (rows == 64 && cols == 64) {
 #pragma unroll
@@ -525,13 +532,22 @@ __device__ __forceinline__ void solve_store(const TileAcc& x, double* g, int64_t
         if (i0 + 4 * q < rows && j0 + 16 * cb < cols) t[4 * q * ld + 16 * cb] = x.c[cb >> 1][cb & 1][q];
   }
 }
-__device__ __forceinline__ void solve_store_sys(const TileAcc& x, double* g) {
-  const int lane = threadIdx.x & 63;
-  double* t = g + (16 * (threadIdx.x >> 6) + (lane >> 4)) * 64 + (lane & 15);
+// Exchange tiles hold X in the order of MFMA operands: element (i, k) of a 64x64
+// tile at x_index(i, k).  Row block i / 16, k steps 2u and 2u + 1 as a pair: one
+// 16-byte load per lane, 1 KB per wave.  Within that KB the rows go in fours,
+// so that a store of the accumulator layout writes two runs of 256 bytes (by row
+// it would be 64-byte pieces, which took the chain 1 us longer per column to
+// complete).
+__device__ __forceinline__ int x_lane(int lane) { return ((lane >> 2) & 3) * 32 + (lane >> 4) * 8 + (lane & 3) * 2; }
+__device__ __forceinline__ int x_index(int i, int k) {
+  return (i >> 4) * 1024 + (k >> 3) * 128 + x_lane((i & 15) + 16 * (k & 3)) + ((k >> 2) & 1);
+}
+__device__ __forceinline__ void solve_store_x(const TileAcc& x, double* g, int w, int lane) {
+  double* t = g + x_index(16 * w + (lane >> 4), lane & 15);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) st_sys(t + 4 * q * 64 + 16 * cb, x.c[cb >> 1][cb & 1][q]);
+    for (int q = 0; q < 4; ++q) st_sys(t + 32 * q + 256 * cb, x.c[cb >> 1][cb & 1][q]);
 }
 
 // Chain: store the factored diagonal tile k held in sA (L_kk) / sB (inverse).
@@ -623,7 +639,7 @@ __device__ __forceinline__ f64x4 block_load(const double* __restrict__ g, int ld
 //   4. factors the rest of C(k+1, k+1), stores its inverse and publishes it at
 //      once (the helpers' solves of column k+1 wait for it).  The log pivots of
 //      tile k are taken by wave 3 beside the last 16x16 factorization.
-// Measured on MI355X at b = 417, us per column: 15.2, against 20.7 with both
+// Measured on MI355X at b = 417, us per column: 15.1, against 20.7 with both
 // products as 32 x 32 quadrants one after the other, X published behind them, L
 // stored and the logarithms taken before the next wait, and the 16x16 blocks
 // factored by column.
@@ -631,7 +647,6 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
                            int* ok_sh) {
   const int nT = p.nT;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int li = lane & 15, lk = lane >> 4;
   {
     int rows, cols;
     const double* g = flow_tile(p, 0, 0, rows, cols);
@@ -660,6 +675,7 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
     // across the columns
     int ln = lane;
     asm volatile("" : "+v"(ln));
+    const int li = ln & 15, lk = ln >> 4;
     if (k > 0) {
       if (!ready && !flow_wait2(p, hflag(p, k, 0), hflag(p, k, 1), tag, ok_sh) && threadIdx.x == 0) atomicOr(p.err, 2);
       // final values, read by nobody on this XCD before: ordinary loads
@@ -667,7 +683,7 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
       gd = hdiag(p, k + 1);
       ld = 64;
     }
-    // C rows 16w .. 16w+15 as pairs: row 2q + lane / 32, columns 2 (lane % 32), +1
+    // C rows 16w .. 16w+15 as pairs: row 2q + ln / 32, columns 2 (ln % 32), +1
     double c[16];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -680,18 +696,18 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
     f64x4 d2 = block_load(gd, ld, rows, bi2, bj2, ln);
     // while those loads are in flight: L_kk out of sA
     chain_store_l(p, k, sA);
-    const double lii = sA[lane * BTA_LDS_LD + lane];
+    const double lii = sA[ln * BTA_LDS_LD + ln];
     if (threadIdx.x == 0) ok_sh[1] = 0;  // waves whose stores of X have completed
     lds_barrier();
     // the wave's rows of C through its own rows of sA into MFMA operands
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const int r = 16 * w + 2 * q + (lane >> 5);
+      const int r = 16 * w + 2 * q + (ln >> 5);
       const bool in = r < rows;
-      *(f64x2*)&sA[r * BTA_LDS_LD + 2 * (lane & 31)] = f64x2{in ? c[2 * q] : 0.0, in ? c[2 * q + 1] : 0.0};
+      *(f64x2*)&sA[r * BTA_LDS_LD + 2 * (ln & 31)] = f64x2{in ? c[2 * q] : 0.0, in ? c[2 * q + 1] : 0.0};
     }
     TileAcc x;
-    tile_solve(x, sA, sB);
+    tile_solve(x, sA, sB, w, ln);
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
@@ -711,11 +727,12 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
     } else {
       // X to the exchange tile: the wave's rows, and a third of wave 0's
       double* xt = xtile(p, k + 1, k);
-      solve_store_sys(x, xt);
+      solve_store_x(x, xt, w, ln);
 #pragma unroll
-      for (int h = 0; h < 6; ++h) {
-        const int r = min(w - 1 + 3 * h, 15);
-        st_sys(xt + r * 64 + ln, sA[r * BTA_LDS_LD + ln]);
+      for (int h = 0; h < 6; ++h) {  // 4 x 16 pieces, as above
+        const int q = min(w - 1 + 3 * h, 15);
+        const int r = 4 * (q & 3) + (ln >> 4), c16 = 16 * (q >> 2) + (ln & 15);
+        st_sys(xt + x_index(r, c16), sA[r * BTA_LDS_LD + c16]);
       }
 #pragma unroll
       for (int t = 0; t < 16; ++t) {
@@ -733,16 +750,10 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       __builtin_amdgcn_s_waitcnt(0);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      if (lane == 0 && atomicAdd(&ok_sh[1], 1) == 2)
+      if (ln == 0 && atomicAdd(&ok_sh[1], 1) == 2)
         __hip_atomic_store(xflag(p, k + 1, k), tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      // ... and to the factor
-      solve_store(x, gx, p.b, rows, 64);
-#pragma unroll
-      for (int h = 0; h < 6; ++h) {
-        const int r = min(w - 1 + 3 * h, min(15, rows - 1));
-        gview(gx)[(unsigned)(r * p.b + ln)] = sA[r * BTA_LDS_LD + ln];
-      }
     }
+    solve_store(x, gx, p.b, rows, 64, w, ln);  // ... and to the factor
     lds_barrier();  // X in sA and inv(L_kk) in sB are no longer read
     if (w == 0) {
       if (mv == 64) store_chol16(d0, e0, sA, sB, 0);
@@ -774,185 +785,282 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
   if (w == 0) chain_log(p, nT - 1, sA[lane * BTA_LDS_LD + lane]);
 }
 
-// One step of a helper: a task, or one column kk of a next-block task.
+// One 64-column product of a helper: its operand tiles and the flags they wait
+// for (f2: nullptr if one tile is both).
 struct HStep {
-  int t, kk;            // task index, column (FLOW_NEXT: current column of the span)
-  int op, rho, c, k;    // decoded task
-  const double* srcA;   // operand tiles (64 x 64, contiguous); TRSM: A is the accumulator
-  const double* srcB;
+  const double* a;
+  const double* b;
   unsigned long long* f1;
   unsigned long long* f2;
 };
 
-__device__ __forceinline__ void next_rows(const FlowArgs& p, int rho, int c, int& ra, int& rb) {
-  const int nT = p.nT;
-  if (rho < nT) { ra = nT + rho; rb = nT + c; }
-  else if (rho == nT) { ra = nT + p.nTL; rb = nT + c; }
-  else { ra = rb = nT + p.nTL; }
+__device__ __forceinline__ HStep step_of(const FlowArgs& p, int ra, int rb, int k) {
+  return HStep{xtile(p, ra, k), xtile(p, rb, k), xflag(p, ra, k), ra != rb ? xflag(p, rb, k) : nullptr};
 }
 
-// Decodes task t at column kk (kk < 0: the task's first column).
-__device__ __forceinline__ HStep make_step(const FlowArgs& p, int t, int kk) {
-  HStep st;
-  st.t = t;
-  flow_decode(p.tasks[t], st.op, st.rho, st.c, st.k);
-  st.kk = kk < 0 ? st.k : kk;
-  st.srcA = st.srcB = nullptr;
-  st.f1 = st.f2 = nullptr;
-  if (st.op == FLOW_UPD) {
-    st.srcA = xtile(p, st.rho, st.k);
-    st.srcB = xtile(p, st.c, st.k);
-    st.f1 = xflag(p, st.rho, st.k);
-    if (st.rho != st.c) st.f2 = xflag(p, st.c, st.k);
-  } else if (st.op == FLOW_TRSM) {
-    st.srcB = p.winv + (int64_t)st.k * 4096;
-    st.f1 = wflag(p, st.k);
-  } else if (st.op == FLOW_NEXT) {
-    int ra, rb;
-    next_rows(p, st.rho, st.c, ra, rb);
-    st.srcA = xtile(p, ra, st.kk);
-    st.srcB = xtile(p, rb, st.kk);
-    st.f1 = xflag(p, ra, st.kk);
-    if (rb != ra) st.f2 = xflag(p, rb, st.kk);
+// A task: op, tile (rho, c), column k.
+struct HTask {
+  int op, rho, c, k;
+};
+
+// The task words are uniform and constant for the launch: scalar loads, so that
+// everything decoded stays in scalar registers and reading ahead in the list
+// waits for no vector load.
+__device__ __forceinline__ HTask task_at(const FlowArgs& p, int t) {
+  HTask h;
+  flow_decode(((const __attribute__((address_space(4))) uint32_t*)p.tasks)[t], h.op, h.rho, h.c, h.k);
+  return h;
+}
+
+// Half of a product's operands (K = 32) of one wave, as MFMA operands: its two
+// row blocks of either tile, k steps 2u and 2u + 1 of the half in element u.
+struct StepHalf {
+  f64x2 a[2][4], b[2][4];
+  // The exchange tiles are written once per launch (before their flag), so
+  // ordinary cached loads after the flag see them; the L2 lines cannot be older
+  // than the launch.
+  __device__ __forceinline__ void load(const HStep& st, int w, int lane, int half) {
+    const gdouble* pa = gview(st.a) + ((w >> 1) * 2048 + half * 512);
+    const gdouble* pb = gview(st.b) + ((w & 1) * 2048 + half * 512);
+    const unsigned at = x_lane(lane);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        a[x][u] = *(const gf64x2*)(pa + (x * 1024 + u * 128) + at);
+        b[x][u] = *(const gf64x2*)(pb + (x * 1024 + u * 128) + at);
+      }
   }
-  return st;
+  // acc -= A B^T over the half
+  __device__ __forceinline__ void mma(TileAcc& t) const {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        t.c[0][0] = mfma_f64_nega(a[0][u][e], b[0][u][e], t.c[0][0]);
+        t.c[0][1] = mfma_f64_nega(a[0][u][e], b[1][u][e], t.c[0][1]);
+        t.c[1][0] = mfma_f64_nega(a[1][u][e], b[0][u][e], t.c[1][0]);
+        t.c[1][1] = mfma_f64_nega(a[1][u][e], b[1][u][e], t.c[1][1]);
+      }
+  }
+};
+
+// The wave waits for the flags of a product (lanes 0 and 1 poll one each).
+__device__ __forceinline__ void step_wait(const FlowArgs& p, const HStep& st, int lane, unsigned long long tag) {
+  const int ok = lane < 2 ? flow_poll(p, lane == 0 ? st.f1 : st.f2, tag) : 1;
+  if (__ballot(ok == 0) != 0 && lane == 0) atomicOr(p.err, 4);
+}
+// The flags' values now (even lanes f1, odd lanes f2), to be looked at later.
+__device__ __forceinline__ unsigned long long step_probe(const HStep& st, int lane) {
+  return __hip_atomic_load((lane & 1) && st.f2 ? st.f2 : st.f1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Issue the operand loads of a step into registers.  The exchange tiles and
-// tile inverses are written once per launch (before their flag), so ordinary
-// cached loads after the flag see them; the L2 lines cannot be older than the
-// launch.
-__device__ __forceinline__ void step_fetch(const HStep& st, TilePrefetch& pa, TilePrefetch& pb) {
-  if (st.srcA) pa.load_full(st.srcA);
-  if (st.srcB && st.srcB != st.srcA) pb.load_full(st.srcB);
+// A helper's target tile in memory, accumulator layout.  Full tiles (all but
+// the last of a ragged size): loads back to back, not waited for here.
+__device__ __forceinline__ void target_load(TileAcc& t, const double* __restrict__ g, int ld, int rows, int cols, int w,
+                                            int lane) {
+  const int r0 = (w >> 1) * 32 + (lane >> 4), c0 = (w & 1) * 32 + (lane & 15);
+  if (rows == 64 && cols == 64) {
+    const unsigned at = r0 * ld + c0;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) t.c[x][y][r] = (gview(g) + ((16 * x + 4 * r) * ld + 16 * y))[at];
+  } else {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          const int i = r0 + 16 * x + 4 * r, j = c0 + 16 * y;
+          const double v = gview(g)[(unsigned)(min(i, rows - 1) * ld + min(j, cols - 1))];
+          t.c[x][y][r] = i < rows && j < cols ? v : 0.0;
+        }
+  }
+}
+__device__ __forceinline__ void target_store(const TileAcc& t, double* __restrict__ g, int ld, int rows, int cols,
+                                             int w, int lane) {
+  const int r0 = (w >> 1) * 32 + (lane >> 4), c0 = (w & 1) * 32 + (lane & 15);
+  const unsigned at = r0 * ld + c0;
+  if (rows == 64 && cols == 64) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) (gview(g) + ((16 * x + 4 * r) * ld + 16 * y))[at] = t.c[x][y][r];
+  } else {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+          if (r0 + 16 * x + 4 * r < rows && c0 + 16 * y < cols)
+            (gview(g) + ((16 * x + 4 * r) * ld + 16 * y))[at] = t.c[x][y][r];
+  }
 }
 
-__device__ __forceinline__ void flow_helper(const FlowArgs& p, int h, unsigned long long tag, double* sA, double* sB,
-                            int* ok_sh) {
+// ... and a hand-off tile in its buffer (64 x 64), past the caches.
+__device__ __forceinline__ void hand_load(TileAcc& t, const double* __restrict__ g, int w, int lane) {
+  const double* at = g + ((w >> 1) * 32 + (lane >> 4)) * 64 + (w & 1) * 32 + (lane & 15);
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) t.c[x][y][r] = ld_sys(at + (16 * x + 4 * r) * 64 + 16 * y);
+}
+__device__ __forceinline__ void hand_store(const TileAcc& t, double* __restrict__ g, int w, int lane) {
+  double* at = g + ((w >> 1) * 32 + (lane >> 4)) * 64 + (w & 1) * 32 + (lane & 15);
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) st_sys(at + (16 * x + 4 * r) * 64 + 16 * y, t.c[x][y][r]);
+}
+
+// Helper h runs its task list.  The operands of an update come from the exchange
+// tiles in MFMA operand order straight into registers: no LDS, and no barrier
+// between the four waves, each of which polls, loads and multiplies its 32 x 32
+// quadrant on its own.  A run of updates of one tile (the columns of a
+// next-block task, or consecutive updates and then the solve of a panel tile)
+// keeps the tile in registers.
+// Up to b = 1600 nothing waits for it but the chain; beyond, it is bound by the
+// waits for tiles of other helpers (the matrix cores are busy 60 % of a launch at
+// b = 2000).  Measured on MI355X, against operands staged through LDS with two
+// barriers per product: b = 1600 445 -> 379 us per block (the chain's own time),
+// b = 2000 770 -> 638, a pair of factorizations at b = 2000 1125 -> 1026; with the
+// task costs above and the exchange order of fours 359, 542 and 872.
+// Loading the next product's first half during the second, or the next task's
+// target during the last product, is slower (655-690): the loads then queue
+// ahead of those that a waiting helper needs first.
+__device__ __forceinline__ void flow_helper(const FlowArgs& p, int h, unsigned long long tag, double* sA, double* sB) {
   const int nT = p.nT;
-  const int t0 = p.off[h], t1 = p.off[h + 1];
-  TileAcc acc;
-  TilePrefetch pa, pb;
-  int carry_rho = -1, carry_c = -1;  // in-panel tile currently held in acc
-  bool fetched = false;              // operands of `cur` already in pa / pb
-  if (t0 >= t1) return;
-  HStep cur = make_step(p, t0, -1);
-  for (;;) {
-    int rows = 0, cols = 0;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const auto* off = (const __attribute__((address_space(4))) int*)p.off;
+  const int t1 = off[h + 1];
+  int t = off[h];
+  while (t < t1) {
+    // opaque, so that the addresses below are formed here and not kept (spilled)
+    // from run to run
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    HTask cur = task_at(p, t);
+    int rows = 0, cols = 0, ld = p.b;
     double* g = nullptr;
-    if (cur.op != FLOW_NEXT) g = flow_tile(p, cur.rho, cur.c, rows, cols);
-    if (cur.op == FLOW_ZERO) {
-      const int cc = threadIdx.x & 63;
-      for (int r = threadIdx.x >> 6; r < rows; r += 4)
-        if (cc < cols) g[(int64_t)r * p.b + cc] = 0.0;
-      if (cur.t + 1 >= t1) break;
-      cur = make_step(p, cur.t + 1, -1);
-      fetched = false;
-      continue;
-    }
-    // accumulator of the step's target: its data come from this helper's own
-    // earlier steps, so its loads are issued before the wait for the operands
-    // and their latency overlaps it
-    double* tg = g;
-    int64_t ld = p.b;
-    int trows = rows, tcols = cols;
-    bool hand = false;
+    int ra = cur.rho, rb = cur.c;  // operand tile rows of an update
     if (cur.op == FLOW_NEXT) {
       if (cur.rho < nT) {
-        tg = p.Dn + (int64_t)(64 * cur.rho) * p.b + 64 * cur.c;
-        trows = min(64, p.b - 64 * cur.rho);
-        tcols = min(64, p.b - 64 * cur.c);
+        g = p.Dn + (int64_t)(64 * cur.rho) * p.b + 64 * cur.c;
+        rows = min(64, p.b - 64 * cur.rho);
+        cols = min(64, p.b - 64 * cur.c);
+        ra = nT + cur.rho;
+        rb = nT + cur.c;
       } else if (cur.rho == nT) {
-        tg = p.Bn + 64 * cur.c;
-        trows = p.a;
-        tcols = min(64, p.b - 64 * cur.c);
+        g = p.Bn + 64 * cur.c;
+        rows = p.a;
+        cols = min(64, p.b - 64 * cur.c);
+        ra = nT + p.nTL;
+        rb = nT + cur.c;
       } else {
-        tg = p.T;
-        ld = p.a;
-        trows = tcols = p.a;
+        g = p.T;
+        rows = cols = ld = p.a;
+        ra = rb = nT + p.nTL;
       }
-      if (cur.kk == cur.k) acc_load(acc, tg, ld, trows, tcols);
     } else {
-      hand = (cur.op == FLOW_UPD) && flow_is_handoff(nT, cur.rho, cur.c);
-      if (!(carry_rho == cur.rho && carry_c == cur.c)) {
-        if (hand && cur.k > 0) acc_load_sys(acc, cur.rho == cur.c ? hdiag(p, cur.c) : hsub(p, cur.c));
-        else acc_load(acc, g, p.b, rows, cols);
+      g = flow_tile(p, cur.rho, cur.c, rows, cols);
+      if (cur.op == FLOW_ZERO) {
+        for (int r = w; r < rows; r += 4)
+          if (lane < cols) g[(int64_t)r * p.b + lane] = 0.0;
+        ++t;
+        continue;
       }
     }
-    if (!fetched) {
-      if (!flow_wait2(p, cur.f1, cur.f2, tag, ok_sh) && threadIdx.x == 0) atomicOr(p.err, 4);
-      step_fetch(cur, pa, pb);
-    }
-    // the following step.  Thread 0 issues the loads of its flags now, both
-    // at once, so that their latency overlaps the staging of this step.
-    HStep nxt;
-    bool has_next = true;
-    if (cur.op == FLOW_NEXT && cur.kk + 1 < flow_next_end(cur.k, nT)) nxt = make_step(p, cur.t, cur.kk + 1);
-    else if (cur.t + 1 < t1) nxt = make_step(p, cur.t + 1, -1);
-    else has_next = false;
-    const bool probe = has_next && nxt.op != FLOW_ZERO;
-    unsigned long long fv1 = 0, fv2 = 0;
-    if (threadIdx.x == 0 && probe) {
-      fv1 = flag_value(nxt.f1, tag);
-      fv2 = flag_value(nxt.f2, tag);
-    }
-    // stage operands in LDS
-    if (cur.op == FLOW_TRSM) acc_to_lds(acc, sA);
-    else pa.store_full(sA);
-    if (cur.srcB != cur.srcA) pb.store_full(sB);
-    // the following step's operands are fetched now if they are ready
-    if (threadIdx.x == 0) *ok_sh = (probe && fv1 == tag && fv2 == tag) ? 1 : 0;
-    lds_barrier();
-    fetched = (*ok_sh != 0);
-    // not ready yet: thread 0 loads the flags again now and looks at them
-    // after the MFMAs (a second chance to fetch ahead of the next step)
-    const bool second = probe && !fetched;
-    unsigned long long gv1 = 0, gv2 = 0;
-    if (second && threadIdx.x == 0) {
-      gv1 = flag_value(nxt.f1, tag);
-      gv2 = flag_value(nxt.f2, tag);
-    }
-    // an update followed by an update: its operand loads ride in the MFMA loop
-    const bool pf_mma = fetched && cur.op != FLOW_TRSM && nxt.srcA != nullptr;
-    if (fetched && !pf_mma) step_fetch(nxt, pa, pb);
-    const double* sBop = (cur.srcB == cur.srcA) ? sA : sB;
+    TileAcc acc;
+    const bool hand = cur.op == FLOW_UPD && flow_is_handoff(nT, cur.rho, cur.c);
+    double* hb = cur.rho == cur.c ? hdiag(p, cur.c) : hsub(p, cur.c);
     if (cur.op == FLOW_TRSM) {
-      tile_solve(acc, sA, sB);  // the accumulator was staged in sA: reuse its registers
-      lds_barrier();
-      solve_store(acc, g, p.b, rows, cols);
-      solve_store_sys(acc, xtile(p, cur.rho, cur.c));
-      carry_rho = carry_c = -1;
-      flow_publish(xflag(p, cur.rho, cur.c), tag);
+      target_load(acc, g, ld, rows, cols, w, lane);
     } else {
-      if (pf_mma) mma_nt64_neg_pf(acc, sA, sBop, pa.r, nxt.srcA, pb.r, nxt.srcB);
-      else mma_nt64<true>(acc, sA, sBop);
-      lds_barrier();
-      if (cur.op == FLOW_NEXT) {
-        if (!(has_next && nxt.op == FLOW_NEXT && nxt.t == cur.t)) acc_store(acc, tg, ld, trows, tcols);
-        carry_rho = carry_c = -1;
-      } else if (hand) {
-        // hand-off tiles are never carried: every update goes to the buffer
-        acc_store_sys(acc, cur.rho == cur.c ? hdiag(p, cur.c) : hsub(p, cur.c));
-        carry_rho = carry_c = -1;
-        if (cur.rho == cur.c + 1 && cur.k == cur.c - 1) flow_publish(hflag(p, cur.c, 0), tag);
-        else if (cur.rho == cur.c && cur.k == cur.c - 2) flow_publish(hflag(p, cur.c - 1, 1), tag);
-      } else if (has_next && nxt.rho == cur.rho && nxt.c == cur.c &&
-                 (nxt.op == FLOW_UPD || nxt.op == FLOW_TRSM)) {
-        carry_rho = cur.rho;  // the next task on this tile keeps the accumulator
-        carry_c = cur.c;
-      } else {
-        acc_store(acc, g, p.b, rows, cols);
-        carry_rho = carry_c = -1;
+      int k = cur.k;
+      const int kend = cur.op == FLOW_NEXT ? flow_next_end(cur.k, nT) : k + 1;
+      HStep st = step_of(p, ra, rb, k);
+      unsigned long long fv = step_probe(st, lane);
+      // (a hand-off tile's buffer holds earlier writes of this workgroup only,
+      // which went past the caches)
+      if (hand && cur.k > 0) hand_load(acc, hb, w, lane);
+      else target_load(acc, g, ld, rows, cols, w, lane);
+      StepHalf h0, h1;
+      if (__ballot(fv != tag) != 0) step_wait(p, st, lane, tag);
+      for (;;) {
+        h0.load(st, w, lane, 0);
+        h1.load(st, w, lane, 1);
+        // the next column of the run (hand-off tiles are never carried: every
+        // update goes to the buffer)
+        if (cur.op == FLOW_NEXT && k + 1 < kend) {
+          ++k;
+        } else {
+          k = -1;
+          ++t;
+          if (cur.op == FLOW_UPD && !hand && t < t1) {
+            const HTask nx = task_at(p, t);
+            if (nx.op == FLOW_UPD && nx.rho == cur.rho && nx.c == cur.c) k = nx.k;
+          }
+          if (k < 0) break;
+        }
+        st = step_of(p, ra, rb, k);
+        fv = step_probe(st, lane);
+        h0.mma(acc);
+        h1.mma(acc);
+        if (__ballot(fv != tag) != 0) step_wait(p, st, lane, tag);
+      }
+      h0.mma(acc);
+      h1.mma(acc);
+      bool solve = false;  // the tile's solve follows
+      if (cur.op == FLOW_UPD && !hand && t < t1) {
+        const HTask nx = task_at(p, t);
+        solve = nx.op == FLOW_TRSM && nx.rho == cur.rho && nx.c == cur.c;
+      }
+      if (!solve) {
+        if (hand) {
+          hand_store(acc, hb, w, lane);
+          if (cur.rho == cur.c + 1 && cur.k == cur.c - 1) flow_publish(hflag(p, cur.c, 0), tag);
+          else if (cur.rho == cur.c && cur.k == cur.c - 2) flow_publish(hflag(p, cur.c - 1, 1), tag);
+        } else {
+          target_store(acc, g, ld, rows, cols, w, lane);
+        }
+        continue;
       }
     }
-    if (second) {  // ok_sh[1] is written once per step, after a barrier that follows its last read
-      if (threadIdx.x == 0) ok_sh[1] = (gv1 == tag && gv2 == tag) ? 1 : 0;
-      lds_barrier();
-      fetched = (ok_sh[1] != 0);
-      if (fetched) step_fetch(nxt, pa, pb);
-    }
-    if (!has_next) break;
-    cur = nxt;
+    // the solve of tile (rho, c)
+    ++t;
+    const double* wi = p.winv + (int64_t)cur.c * 4096;
+    step_wait(p, HStep{wi, nullptr, wflag(p, cur.c), nullptr}, lane, tag);
+    f64x2 iv[8];  // rows 16w + lane / 32 + 2q, columns 2 (lane % 32), +1
+    const unsigned ia = (16 * w + (lane >> 5)) * 64 + 2 * (lane & 31);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) iv[q] = *(const gf64x2*)(gview(wi) + (128 * q) + ia);
+    // (the barrier of the last solve's publication: sA and sB are free)
+    double* sc = sA + ((w >> 1) * 32 + (lane >> 4)) * BTA_LDS_LD + (w & 1) * 32 + (lane & 15);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[(16 * x + 4 * r) * BTA_LDS_LD + 16 * y] = acc.c[x][y][r];
+    double* si = sB + (16 * w + (lane >> 5)) * BTA_LDS_LD + 2 * (lane & 31);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) *(f64x2*)(si + 2 * q * BTA_LDS_LD) = iv[q];
+    lds_barrier();
+    tile_solve(acc, sA, sB, w, lane);
+    solve_store(acc, g, p.b, rows, cols, w, lane);
+    solve_store_x(acc, xtile(p, cur.rho, cur.c), w, lane);
+    flow_publish(xflag(p, cur.rho, cur.c), tag);
   }
 }
 
@@ -962,7 +1070,7 @@ __global__ void __launch_bounds__(BTA_THREADS, 2) k_panel_flow(FlowArgs p) {
   __shared__ int ok_sh[2];
   const unsigned long long tag = (p.epoch[0] << 20) | (unsigned long long)p.blk;
   if (blockIdx.x == 0) flow_chain(p, tag, sA, sB, ok_sh);
-  else flow_helper(p, blockIdx.x - 1, tag, sA, sB, ok_sh);
+  else flow_helper(p, blockIdx.x - 1, tag, sA, sB);
 }
 
 // -------------------------------------------------------------------- host
@@ -1125,7 +1233,7 @@ __global__ void __launch_bounds__(BTA_THREADS, 2) k_panel_flow_batched(FlowBatch
   const FlowArgs p = fb.e[lo];
   const unsigned long long tag = (p.epoch[0] << 20) | (unsigned long long)p.blk;
   if (local == 0) flow_chain(p, tag, sA, sB, ok_sh);
-  else flow_helper(p, local - 1, tag, sA, sB, ok_sh);
+  else flow_helper(p, local - 1, tag, sA, sB);
 }
 
 void flow_launch_batched(const FlowBatch& fb, int total, hipStream_t st) {
