@@ -175,20 +175,21 @@ int bta_logdet(bta_ws_t ws, const double* D, const double* T, int n, int b, int 
  * concurrently per wave (taken from the first problem's workspace; 0 = 6,
  * at most 8). */
 #define BTA_OPT_BATCH_LANES 6
-/* Selected inversion: 1 (default) = the b x b x b products
+/* Selected inversion: 1 (default) = for b > 1600 the b x b x b products
  * Sigma_{i+1,i} = -Sigma_{i+1,i+1} G_i as rocBLAS dgemm calls on the caller's
  * stream (not while that stream is under graph capture), 0 = the grouped
- * FP64-MFMA kernel for every product. */
+ * FP64-MFMA kernels for every product. */
 #define BTA_OPT_BLAS 7
 /* Persistent panel: the near-diagonal tiles ((c,c), (c+1,c), (c+2,c)), whose
  * updates and solves the chain waits for, go to a pool of helpers / value
  * helpers (at least min(10, helpers / 8)) that own nothing else (default 16;
  * 1..64). */
 #define BTA_OPT_FLOW_NEAR 8
-/* 64x64 grouped GEMM main loop: 0 (default) = one LDS buffer, the next K
- * chunk loaded into registers while the current one is multiplied; 1 = two
- * LDS buffers with loads issued two K chunks ahead (slower on MI355X: 470 us
- * against 395 us for NN 2000^3; kept for comparison). */
+/* Grouped GEMM main loop: 0 (default) = by the launch's tile counts and
+ * operand forms, operands loaded straight into registers (32x32 or 64x64
+ * tiles) or staged through one LDS buffer (triangular products); 1 = 64x64
+ * tiles through two LDS buffers with loads issued two K chunks ahead (slower
+ * on MI355X: 470 us against 262 us for NN 2000^3; kept for comparison). */
 #define BTA_OPT_GEMM_KERNEL 9
 /* Persistent panel, block update D_{i+1} -= L_i L_i^T, B_{i+1} -= B_i L_i^T,
  * T -= B_i B_i^T: 1 = applied by each block's launch through helper tasks
@@ -236,8 +237,8 @@ int bta_potrs(bta_ws_t ws, double* D, double* L, double* B, double* T, int n, in
  * symmetric), L[i] <- Sigma_{i+1,i}, B[i] <- Sigma_{n,i}, T <- Sigma_T.
  * Replaces serinv.pobtasi(D, L, B, T) / pobtsi(D, L) as called by
  * SerinvSolver.selected_inversion (structured_solver.py:168-190).  With
- * BTA_OPT_BLAS on (the default) the Sigma_{i+1,i} products are rocBLAS dgemm
- * calls on `stream`; everything else runs in this library's kernels.  Returns
+ * BTA_OPT_BLAS on (the default) and b > 1600 the Sigma_{i+1,i} products are
+ * rocBLAS dgemm calls on `stream`; everything else runs in this library's kernels.  Returns
  * BTA_E_LIB if a rocBLAS call fails, BTA_E_NORES without BTA_WS_SELINV. */
 int bta_potri(bta_ws_t ws, double* D, double* L, double* B, double* T, int n, int b, int a,
               void* stream);

@@ -1,4 +1,4 @@
-// Grouped FP64 GEMM on 64x64 output tiles (FP64 MFMA), driven by a job table
+// Grouped FP64 GEMM on 32x32 to 128x128 output tiles (FP64 MFMA), driven by a job table
 // in device memory.  One launch covers any number of independent jobs of any
 // shapes; a workgroup finds its job by binary search over the tile prefix
 // sums.  Each job computes
@@ -38,14 +38,6 @@ struct GemmJob {
   int lower;     // 1: only tiles with tr >= tc
   int mirror;    // with lower: also write the transpose into the upper triangle
   int nseg;
-  // split = 2 (lower jobs of the 64-tile kernel only): two workgroups per
-  // output tile, one per half of the tile's K chunks; each writes its partial
-  // sum to part (two 64 x 64 slots per tile) and counts itself in cnt (one
-  // counter per tile, zero between launches), and the second to arrive adds
-  // the other's partial and writes the tile.  Set by DevPlan::build.
-  int split;
-  double* part;
-  int* cnt;
   GemmSeg seg[3];
 };
 
@@ -56,21 +48,23 @@ struct GemmLaunch {
   int ts = 64;              // output tile edge: 64 or 128
   explicit GemmLaunch(int tile = 64) : ts(tile) {}
   int tiles() const { return prefix.empty() ? 0 : prefix.back(); }
+  static int job_tiles(const GemmJob& j, int edge) {
+    const int tm = (j.m + edge - 1) / edge, tn = (j.n + edge - 1) / edge;
+    return j.lower ? tm * (tm + 1) / 2 : tm * tn;
+  }
   void add(const GemmJob& j) {
     if (j.m <= 0 || j.n <= 0) return;
     if (prefix.empty()) prefix.push_back(0);
-    const int tm = (j.m + ts - 1) / ts, tn = (j.n + ts - 1) / ts;
     jobs.push_back(j);
-    prefix.push_back(prefix.back() + (j.lower ? tm * (tm + 1) / 2 : tm * tn) * j.split);
+    prefix.push_back(prefix.back() + job_tiles(j, ts));
   }
 };
 
-// Default output tile edge.  64x64 tiles run two workgroups per CU (one hides
-// the other's load latency) and keep 256 CUs busy down to 2000x2000 outputs;
-// measured on MI355X at b = 2000 and 4500 they beat the 128x128 kernel for
-// every product of the factorization and the selected inversion (1.44x on
-// the selected inversion at b = 2000).  128 stays available to the
-// autotuner.
+// Default output tile edge: 64 (DevPlan::build takes 32 x 32 tiles where a
+// launch has few of them).  Measured on MI355X at b = 2000 and 4500 64x64 tiles
+// beat the 128x128 kernel for every product of the factorization and the
+// selected inversion (1.44x on the selected inversion at b = 2000).  128 stays
+// available to the autotuner.
 inline int pick_tile(int m, int n) {
   (void)m;
   (void)n;
@@ -93,7 +87,7 @@ inline GemmSeg seg(const double* A, int lda, int ta, const double* B, int ldb, i
 }
 
 inline GemmJob job(double* C, int m, int n, int ldc, double beta, int lower = 0, int mirror = 0) {
-  GemmJob j;
+  GemmJob j = {};
   j.C = C;
   j.beta = beta;
   j.m = m;
@@ -102,9 +96,6 @@ inline GemmJob job(double* C, int m, int n, int ldc, double beta, int lower = 0,
   j.lower = lower;
   j.mirror = mirror;
   j.nseg = 0;
-  j.split = 1;
-  j.part = nullptr;
-  j.cnt = nullptr;
   return j;
 }
 
@@ -119,14 +110,11 @@ inline GemmJob& add_seg(GemmJob& j, const GemmSeg& s) {
 struct DevPlan {
   // vec: every operand has an even leading dimension and a 16-byte aligned
   // base (the pipelined kernel's paired loads need both)
-  // split: the launch holds split jobs (run by the 64-tile kernel whatever
-  // the variant asked for)
-  struct Entry { int job_off, pre_off, njobs, tiles, ts, vec, split; };
+  // kernel: GemmKernel of the default variant, its tiles and their prefix sums
+  struct Entry { int job_off, pre_off, njobs, tiles, ts, vec, kernel, kpre_off, ktiles; };
   GemmJob* d_jobs = nullptr;
   int* d_prefix = nullptr;
-  double* d_part = nullptr;  // partial sums of split jobs, shared by the launches (one stream)
-  int* d_cnt = nullptr;      // their per-tile counters
-  size_t bytes = 0;  // device bytes of the job table, prefix sums and split scratch
+  size_t bytes = 0;  // device bytes of the job table and prefix sums
   std::vector<Entry> launches;
   DevPlan() = default;
   DevPlan(const DevPlan&) = delete;

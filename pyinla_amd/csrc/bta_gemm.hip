@@ -53,24 +53,31 @@ __device__ __forceinline__ int find_job(const int* __restrict__ prefix, int njob
 }
 
 // Output tile of workgroup `local` of a tm x tn job.  Workgroups are
-// dispatched to the 8 XCDs round-robin (blockIdx % 8); when the job's tiles
-// start on an XCD boundary and split evenly, XCD x takes a contiguous run of
-// the tiles ordered in bands of 8 tile rows (column by column inside a band),
-// i.e. a compact 8 x (T/64) rectangle whose A and B panels its L2 shares.
-#ifndef BTA_GEMM_XCD
-#define BTA_GEMM_XCD 1
-#endif
-__device__ __forceinline__ void xcd_tile(int local, int first, int tm, int tn, int& tr, int& tc) {
-  const int T = tm * tn;
-  int t = local;
-  if (BTA_GEMM_XCD && (first & 7) == 0 && (T & 7) == 0 && tm % 8 == 0) t = (local & 7) * (T >> 3) + (local >> 3);
-  if (BTA_GEMM_XCD && tm % 8 == 0) {
-    const int band = t / (8 * tn), idx = t % (8 * tn);
-    tr = band * 8 + (idx & 7);
-    tc = idx >> 3;
-  } else {
+// dispatched to the 8 XCDs round-robin (blockIdx % 8), so the tiles are put in
+// an order and XCD x takes the x-th eighth of it: a compact region whose A and
+// B panels its L2 shares.  The order is bands of 8 tile rows, column by column,
+// where all tiles have the same K; where K depends on the tile column or row
+// (triangular operand) every XCD takes whole rows or columns of tiles, or the
+// XCDs' shares differ by up to 3:1 (L W at b = 2000, 12 blocks in a launch:
+// 210 us per block in bands, 160 by rows).
+__device__ __forceinline__ int xcd_share(int local, int T) {
+  const int x = local & 7, r = T & 7;
+  return x * (T >> 3) + min(x, r) + (local >> 3);
+}
+__device__ __forceinline__ void xcd_tile(int local, int tm, int tn, int tri, int& tr, int& tc) {
+  const int t = xcd_share(local, tm * tn);
+  const bool ka = tri & (TRI_A_LOWER | TRI_A_UPPER), kb = tri & (TRI_B_LOWER | TRI_B_UPPER);
+  if (kb && !ka) {
     tr = t / tn;
     tc = t % tn;
+  } else if (ka && !kb) {
+    tc = t / tm;
+    tr = t % tm;
+    if (tri & TRI_A_LOWER) tr = tm - 1 - tr;  // longest K first
+  } else {
+    const int band = t / (8 * tn), idx = t - band * 8 * tn, h = min(8, tm - 8 * band);
+    tr = 8 * band + idx % h;
+    tc = idx / h;
   }
 }
 
@@ -154,17 +161,14 @@ __global__ void __launch_bounds__(BTA_THREADS, BTA_GEMM_MINB) k_gemm_grouped(con
                                                              const int* __restrict__ prefix, int njobs) {
   __shared__ double sA[64 * BTA_GEMM_LD];
   __shared__ double sB[64 * BTA_GEMM_LD];
-  __shared__ int last_sh;
   const int jid = find_job(prefix, njobs, blockIdx.x);
   const GemmJob& g = jobs[jid];
-  const bool split = g.split == 2;
-  const int local = split ? (blockIdx.x - prefix[jid]) >> 1 : blockIdx.x - prefix[jid];
-  const int half = split ? (blockIdx.x - prefix[jid]) & 1 : 0;
+  const int local = blockIdx.x - prefix[jid];
   int tr, tc;
   if (g.lower) decode_lower(local, tr, tc);
   else {
     const int tm = (g.m + 63) / 64, tn = (g.n + 63) / 64;
-    xcd_tile(local, prefix[jid], tm, tn, tr, tc);
+    xcd_tile(local, tm, tn, g.seg[0].tri, tr, tc);
   }
   const int rows = min(64, g.m - tr * 64), cols = min(64, g.n - tc * 64);
   // A tile at a ragged edge of a job at least 64 wide works on the 64-wide
@@ -179,7 +183,7 @@ __global__ void __launch_bounds__(BTA_THREADS, BTA_GEMM_MINB) k_gemm_grouped(con
   const int wrows = min(64, g.m - r0), wcols = min(64, g.n - c0);
   double* ct = g.C + (int64_t)r0 * g.ldc + c0;
   TileAcc acc;
-  if (g.beta != 0.0 && half == 0) {  // the second half of a split tile starts from zero
+  if (g.beta != 0.0) {
     acc_load(acc, ct, g.ldc, wrows, wcols);
     if (g.beta != 1.0) {
 #pragma unroll
@@ -231,23 +235,7 @@ __global__ void __launch_bounds__(BTA_THREADS, BTA_GEMM_MINB) k_gemm_grouped(con
     if (sg.tb == 1) pb.load(sg.B + (int64_t)c0 * sg.ldb + k0, sg.ldb, 0, wcols, kw, mb, c0, k0);
     else pb.load(sg.B + (int64_t)k0 * sg.ldb + c0, sg.ldb, 1, wcols, kw, mb, c0, k0);
   };
-  // a split tile's halves take the first ceil(nch / 2) and the remaining of
-  // its nch chunks
-  int qend = 0x7fffffff;
-  int q = 0;
-  if (split) {
-    int nch = 0;
-    for (int sid = 0; sid < g.nseg; ++sid) {
-      int kb, ke;
-      seg_range(sid, kb, ke);
-      if (ke > kb) nch += (ke - kb + BTA_GEMM_KC - 1) / BTA_GEMM_KC;
-    }
-    qend = half ? nch : (nch + 1) / 2;
-  }
   bool have = (g.nseg > 0) && next_chunk(true);
-  if (half)
-    for (const int q0 = qend - qend / 2; have && q < q0; ++q) have = next_chunk(false);
-  if (q >= qend) have = false;
   if (have) fetch();
   while (have) {
     const GemmSeg& sg = g.seg[seg_id];
@@ -255,36 +243,10 @@ __global__ void __launch_bounds__(BTA_THREADS, BTA_GEMM_MINB) k_gemm_grouped(con
     pa.store(sA, sg.ta, sg.alpha);
     pb.store(sB, sg.tb == 1 ? 0 : 1);
     __syncthreads();
-    have = next_chunk(false) && ++q < qend;
+    have = next_chunk(false);
     if (have) fetch();
     mma_nt_ld<BTA_GEMM_LD>(acc, sA, sB, (kw + 3) & ~3);
     lds_barrier();  // not a wait for the next chunk's loads: its stores wait for them
-  }
-  if (split) {
-    // both halves publish their partial sums (write-through stores that have
-    // completed before the counter moves); the second to count adds the other
-    // half's partial (a + b == b + a: the tile is the same whichever comes
-    // second), resets the counter for the next launch and writes the tile
-    double* mine = g.part + ((int64_t)local * 2 + half) * 4096;
-    acc_store_sys(acc, mine);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int before = __hip_atomic_fetch_add(g.cnt + local, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      if (before == 1) __hip_atomic_store(g.cnt + local, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      last_sh = before;
-    }
-    __syncthreads();
-    if (last_sh != 1) return;
-    const double* other = g.part + ((int64_t)local * 2 + (half ^ 1)) * 4096;
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int y = 0; y < 2; ++y)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc.c[x][y][r] += ld_sys(&other[acc_row(x, r) * 64 + acc_col(y)]);
   }
   // epilogue
 #pragma unroll
@@ -309,6 +271,12 @@ __global__ void __launch_bounds__(BTA_THREADS, BTA_GEMM_MINB) k_gemm_grouped(con
         }
       }
 }
+
+}  // namespace bta
+
+#include "bta_gemm_direct.h"
+
+namespace bta {
 
 // ------------------------------------------- 64x64 tiles, pipelined K loop
 //
@@ -424,7 +392,7 @@ __global__ void __launch_bounds__(BTA_THREADS, 4) k_gemm_grouped_db(const GemmJo
   if (g.lower) decode_lower(local, tr, tc);
   else {
     const int tm = (g.m + 63) / 64, tn = (g.n + 63) / 64;
-    xcd_tile(local, prefix[jid], tm, tn, tr, tc);
+    xcd_tile(local, tm, tn, g.seg[0].tri, tr, tc);
   }
   const int rows = min(64, g.m - tr * 64), cols = min(64, g.n - tc * 64);
   double* ct = g.C + (int64_t)(tr * 64) * g.ldc + tc * 64;
@@ -731,24 +699,65 @@ DevPlan::~DevPlan() { release(); }
 void DevPlan::release() {
   if (d_jobs) hipFree(d_jobs);
   if (d_prefix) hipFree(d_prefix);
-  if (d_part) hipFree(d_part);
-  if (d_cnt) hipFree(d_cnt);
   d_jobs = nullptr;
   d_prefix = nullptr;
-  d_part = nullptr;
-  d_cnt = nullptr;
   bytes = 0;
   launches.clear();
+}
+
+// Kernels of a launch of 64-wide tiles (BTA_OPT_GEMM_KERNEL 0).
+enum GemmKernel : int {
+  KER_LDS,   // k_gemm_grouped
+  KER_D32,   // k_gemm_direct, 32 x 32 tiles, four waves each with a quarter of K
+  KER_D32W,  // 32 x 32 tiles, one wave each
+  KER_D64,   // 64 x 64 tiles, one wave each
+  KER_D64K   // 64 x 64 tiles, two waves each with a half of K
+};
+
+// The kernel by the number of tiles; times in us of one b x b x b product
+// (NN / lower triangle of TN with mirrored output) measured on MI355X:
+//            b = 417      800        1200       1600        2000       4500
+//   LDS      31 / 31      54 / 53    105 / 81   181 / 131   293 / 228  3070 / 1580
+//   D32      12 / 13      34 / 23    87 / 48    162 / 90    331 / 165
+//   D32W     23 / 25      36 / 37    90 / 60    172 / 117   299 / 154
+//   D64      64 / 66      109 / 112  160 / 163  210 / 212   262 / 263  2845 / 1731
+//   D64K     39 / 41      63 / 64    90 / 91    217 / 117   274 / 271  2895 / 1470
+// One wave per SIMD runs a 64 x 64 tile (1024 at a time), two run 32 x 32 tiles
+// (2048): D64 and D64K are the fastest where their last turn is 85 % full, else
+// the smaller tiles are.  Triangular products have short and uneven K ranges
+// and mask a good part of their chunks: LDS (block inverses, 20 blocks of b =
+// 2000, 512-wide merge: LDS 145 us, D32W 177, D64 204; L W 160 us per block
+// against 165 with D64).  Both operands K-contiguous (A B^T: the block updates
+// of the factorization): LDS too.  32 x 32 tiles run into the half lines there
+// (b = 1600: 244 us against 186), and K in parts changes what the updates
+// round: D_{i+1} - L_i L_i^T cancels, and the coregional model's f moves by
+// 1e-10 of its value.
+static GemmKernel pick_kernel(const GemmLaunch& l) {
+  bool nt = false, mixed = false;
+  int64_t t32 = 0, t64 = 0, tri64 = 0;
+  for (const GemmJob& j : l.jobs) {
+    t32 += GemmLaunch::job_tiles(j, 32);
+    t64 += GemmLaunch::job_tiles(j, 64);
+    if (j.seg[0].tri) tri64 += GemmLaunch::job_tiles(j, 64);
+    for (int q = 0; q < j.nseg; ++q) {
+      const GemmSeg& sg = j.seg[q];
+      nt = nt || (sg.ta == 0 && sg.tb == 1);
+      mixed = mixed || sg.alpha != j.seg[0].alpha;
+    }
+  }
+  // k_gemm_direct scales a job's sum once, with the alpha of its first segment
+  if (mixed || nt || 2 * tri64 > t64) return KER_LDS;
+  auto fill = [](int64_t t, int64_t slots) { return (double)t / (double)((t + slots - 1) / slots * slots); };
+  const double u1 = fill(t64, 1024), u2 = 0.96 * fill(2 * t64, 1024);
+  if (u1 >= 0.85 && u1 >= u2) return KER_D64;
+  if (u2 >= 0.85) return KER_D64K;
+  return t32 <= 700 || fill(t32, 2048) < 0.85 ? KER_D32 : KER_D32W;
 }
 
 int DevPlan::build(const std::vector<GemmLaunch>& ls) {
   release();
   std::vector<GemmJob> all;
   std::vector<int> pre;
-  // split jobs: tile offsets into one scratch shared by all launches (they run
-  // one after another on the plan's stream), sized for the largest launch
-  int64_t split_max = 0;
-  std::vector<int64_t> split_off;
   for (const auto& l : ls) {
     Entry e;
     e.job_off = (int)all.size();
@@ -757,8 +766,6 @@ int DevPlan::build(const std::vector<GemmLaunch>& ls) {
     e.tiles = l.tiles();
     e.ts = l.ts;
     e.vec = 1;
-    e.split = 0;
-    int64_t split_tiles = 0;
     for (const GemmJob& j : l.jobs) {
       for (int q = 0; q < j.nseg; ++q) {
         const GemmSeg& sg = j.seg[q];
@@ -766,57 +773,51 @@ int DevPlan::build(const std::vector<GemmLaunch>& ls) {
             (reinterpret_cast<uintptr_t>(sg.B) & 15))
           e.vec = 0;
       }
-      if (j.split != 1 && (j.split != 2 || !j.lower || l.ts != 64)) return (int)hipErrorInvalidValue;
-      split_off.push_back(j.split == 2 ? split_tiles : -1);
-      if (j.split == 2) {
-        const int tm = (j.m + 63) / 64;
-        split_tiles += tm * (tm + 1) / 2;
-        e.split = 1;
-      }
     }
-    split_max = std::max(split_max, split_tiles);
+    e.kernel = l.ts == 64 ? pick_kernel(l) : KER_LDS;
+    e.kpre_off = e.pre_off;
+    e.ktiles = e.tiles;
+    pre.insert(pre.end(), l.prefix.begin(), l.prefix.end());
+    if (e.kernel == KER_D32 || e.kernel == KER_D32W) {
+      e.kpre_off = (int)pre.size();
+      e.ktiles = 0;
+      for (const GemmJob& j : l.jobs) {
+        pre.push_back(e.ktiles);
+        e.ktiles += GemmLaunch::job_tiles(j, 32);
+      }
+      pre.push_back(e.ktiles);
+    }
     launches.push_back(e);
     all.insert(all.end(), l.jobs.begin(), l.jobs.end());
-    pre.insert(pre.end(), l.prefix.begin(), l.prefix.end());
   }
   if (all.empty()) return 0;
   hipError_t e;
-  if (split_max > 0) {
-    if ((e = hipMalloc(&d_part, (size_t)split_max * 2 * 4096 * sizeof(double))) != hipSuccess) return (int)e;
-    if ((e = hipMalloc(&d_cnt, (size_t)split_max * sizeof(int))) != hipSuccess) return (int)e;
-    if ((e = hipMemset(d_cnt, 0, (size_t)split_max * sizeof(int))) != hipSuccess) return (int)e;
-    for (size_t q = 0; q < all.size(); ++q)
-      if (split_off[q] >= 0) {
-        all[q].part = d_part + split_off[q] * 2 * 4096;
-        all[q].cnt = d_cnt + split_off[q];
-      }
-  }
   if ((e = hipMalloc(&d_jobs, all.size() * sizeof(GemmJob))) != hipSuccess) return (int)e;
   if ((e = hipMalloc(&d_prefix, pre.size() * sizeof(int))) != hipSuccess) return (int)e;
   if ((e = hipMemcpy(d_jobs, all.data(), all.size() * sizeof(GemmJob), hipMemcpyHostToDevice)) != hipSuccess)
     return (int)e;
   if ((e = hipMemcpy(d_prefix, pre.data(), pre.size() * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
     return (int)e;
-  bytes = all.size() * sizeof(GemmJob) + pre.size() * sizeof(int) +
-          (size_t)split_max * (2 * 4096 * sizeof(double) + sizeof(int));
+  bytes = all.size() * sizeof(GemmJob) + pre.size() * sizeof(int);
   return 0;
 }
 
 void DevPlan::launch(int idx, hipStream_t st, int variant) const {
   const Entry& e = launches[idx];
   if (e.tiles <= 0) return;
-  if (e.split)
-    hipLaunchKernelGGL(k_gemm_grouped, dim3(e.tiles), dim3(BTA_THREADS), 0, st, d_jobs + e.job_off,
-                       d_prefix + e.pre_off, e.njobs);
-  else if (e.ts == BIG_TS)
-    hipLaunchKernelGGL(k_gemm_grouped_big, dim3(e.tiles), dim3(BTA_THREADS), 0, st, d_jobs + e.job_off,
-                       d_prefix + e.pre_off, e.njobs);
-  else if (variant == 1 && e.vec)
-    hipLaunchKernelGGL(k_gemm_grouped_db, dim3(e.tiles), dim3(BTA_THREADS), 0, st, d_jobs + e.job_off,
-                       d_prefix + e.pre_off, e.njobs);
-  else
-    hipLaunchKernelGGL(k_gemm_grouped, dim3(e.tiles), dim3(BTA_THREADS), 0, st, d_jobs + e.job_off,
-                       d_prefix + e.pre_off, e.njobs);
+  const GemmJob* jobs = d_jobs + e.job_off;
+  auto run = [&](auto* kernel, int tiles, int threads, int pre_off) {
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(threads), 0, st, jobs, d_prefix + pre_off, e.njobs);
+  };
+  if (e.ts == BIG_TS) return run(k_gemm_grouped_big, e.tiles, BTA_THREADS, e.pre_off);
+  if (variant == 1 && e.vec) return run(k_gemm_grouped_db, e.tiles, BTA_THREADS, e.pre_off);
+  switch (e.kernel) {
+    case KER_D32: return run(k_gemm_direct<1, 4, 4, 2>, e.ktiles, 256, e.kpre_off);
+    case KER_D32W: return run(k_gemm_direct<1, 1, 4, 2>, e.ktiles, 64, e.kpre_off);
+    case KER_D64: return run(k_gemm_direct<2, 1, 3, 1>, e.ktiles, 64, e.kpre_off);
+    case KER_D64K: return run(k_gemm_direct<2, 2, 3, 1>, e.ktiles, 128, e.kpre_off);
+    default: return run(k_gemm_grouped, e.ktiles, BTA_THREADS, e.kpre_off);
+  }
 }
 
 }  // namespace bta

@@ -154,7 +154,7 @@ struct Workspace {
   PotriPlan* potri_cur = nullptr;
   bool graphs_stale = false;        // a plan cache was emptied: drop recorded graphs
   void* blas = nullptr;  // rocblas_handle, created with the first plan that uses it
-  int use_blas = 1;      // 0: grouped kernel for every product
+  int use_blas = 1;      // 0: grouped kernels for every product; 1: see potri_build
   TimingLog* tlog = nullptr;  // non-null: bracket launches with events
   // Output-tile edge per GEMM class: 0 = heuristic (pick_tile), 64 or 128.
   int tile_update = 0;   // block updates of the factorization
@@ -166,7 +166,7 @@ struct Workspace {
   int flow_delta = 0;    // 0: list-scheduled task order; >= 1: level order, far-tile update groups
   int flow_near = 16;    // near pool = helpers / flow_near (see flow_near_pool)
   int flow_fold = 0;     // block update: 0 = automatic, 1 = in the persistent panel, 2 = a grouped GEMM after it
-  int gemm_variant = 0;  // 64x64 grouped GEMM: 0 = single LDS buffer, 1 = two LDS buffers
+  int gemm_variant = 0;  // grouped GEMM: 0 = chosen by pick_kernel, 1 = two LDS buffers
   int batch_lanes = 0;   // problems per wave of a batched factorization (0 = 6)
   // persistent-panel exchange buffers, sized for the workspace's arrowhead
   // (allocated by bta_ws_create when the flow panel can run)
