@@ -282,6 +282,16 @@ int bta_scatter_coo(double* D, double* L, double* B, double* T, const uint64_t* 
                     const double* val, const int* src_idx, int64_t count, double scale,
                     int accumulate, void* stream);
 
+/* Host-side map of a COO pattern into the blocks (no device work): for every
+ * entry e that the scatter places -- both triangles of the diagonal blocks, the
+ * sub-diagonal blocks (i+1, i), with a > 0 the arrow rows and the tip
+ * (structured_solver.py:214-250); lower_only != 0 keeps row >= col only -- in
+ * COO order idx[q] = e and code[q] as above.  rows / cols are host arrays of
+ * nnz 4- or 8-byte integers (index_bytes), idx and code hold nnz entries;
+ * *count receives the number placed. */
+int bta_pattern_codes(const void* rows, const void* cols, int index_bytes, int64_t nnz, int n, int b, int a,
+                      int lower_only, int64_t* idx, uint64_t* code, int64_t* count);
+
 /* out[e] = block entry at code[e]: the gather of the selected inverse on a
  * sparsity pattern (SerinvSolver._structured_to_spmatrix,
  * structured_solver.py:470-538). */

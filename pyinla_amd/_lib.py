@@ -41,6 +41,7 @@ SIGNATURES = {
     "bta_block_inverses": (_I, [_P, _P, _I, _I, _P]),
     "bta_assemble_kron": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P, _P, _I, _P, _D, _P]),
     "bta_scatter_coo": (_I, [_P, _P, _P, _P, _P, _P, _P, C.c_int64, _D, _I, _P]),
+    "bta_pattern_codes": (_I, [_P, _P, _I, C.c_int64, _I, _I, _I, _I, _P, _P, C.POINTER(C.c_int64)]),
     "bta_gather_coo": (_I, [_P, _P, _P, _P, _P, _P, C.c_int64, _P]),
     "bta_bilinear_coo": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int64, _I, _P, _I, _P, _P]),
     "bta_quadform_rows": (_I, [_P, _P, _P, _P, _I, _I, _I, _P, _P, _P, C.c_int64, _P, _P]),

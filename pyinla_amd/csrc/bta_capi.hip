@@ -52,6 +52,57 @@ void TimingLog::end(int cls, hipStream_t st) {
 
 }  // namespace bta
 
+namespace bta {
+
+// One pass over the pattern; the row's block and the row in it come from a
+// product with 1 / b, corrected by one, instead of two integer divisions
+// (350 k entries: 7.6 ms in numpy, 1.4 ms here).
+template <class I>
+int64_t pattern_codes(const I* rows, const I* cols, int64_t nnz, int n, int b, int a, bool lower_only, int64_t* idx,
+                      uint64_t* code) {
+  const int64_t nb = (int64_t)n * b, bb = (int64_t)b * b, ab = (int64_t)a * b;
+  const double inv = 1.0 / b;
+  auto block = [&](int64_t r, int64_t& m) {
+    int64_t q = (int64_t)((double)r * inv);
+    m = r - q * b;
+    if (m < 0) {
+      --q;
+      m += b;
+    } else if (m >= b) {
+      ++q;
+      m -= b;
+    }
+    return q;
+  };
+  int64_t out = 0;
+  for (int64_t e = 0; e < nnz; ++e) {
+    const int64_t r = rows[e], c = cols[e];
+    if (r < 0 || c < 0 || (lower_only && r < c)) continue;
+    uint64_t v;
+    int64_t ri, cj;
+    if (r < nb) {
+      if (c >= nb) continue;
+      const int64_t bi = block(r, ri), bj = block(c, cj);
+      if (bi == bj) v = (uint64_t)(bi * bb + ri * b + cj);
+      else if (bi == bj + 1) v = (1ull << 60) | (uint64_t)(bj * bb + ri * b + cj);
+      else continue;
+    } else {
+      if (r >= nb + a || c >= nb + a) continue;
+      if (c < nb) {
+        const int64_t bj = block(c, cj);
+        v = (2ull << 60) | (uint64_t)(bj * ab + (r - nb) * b + cj);
+      } else {
+        v = (3ull << 60) | (uint64_t)((r - nb) * a + (c - nb));
+      }
+    }
+    idx[out] = e;
+    code[out++] = v;
+  }
+  return out;
+}
+
+}  // namespace bta
+
 namespace {
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
@@ -542,6 +593,19 @@ int bta_ws_reset_timing(bta_ws_t ws) {
   if (!ws || !ws->w.tlog) return BTA_E_ARG;
   hipDeviceSynchronize();
   for (int c = 0; c < bta::KC_COUNT; ++c) ws->w.tlog->used[c] = 0;
+  return 0;
+}
+
+int bta_pattern_codes(const void* rows, const void* cols, int index_bytes, int64_t nnz, int n, int b, int a,
+                      int lower_only, int64_t* idx, uint64_t* code, int64_t* count) {
+  if (nnz < 0 || n < 1 || b < 1 || a < 0 || !count || (index_bytes != 4 && index_bytes != 8)) return BTA_E_ARG;
+  if (nnz > 0 && (!rows || !cols || !idx || !code)) return BTA_E_ARG;
+  if (index_bytes == 4)
+    *count = bta::pattern_codes(static_cast<const int32_t*>(rows), static_cast<const int32_t*>(cols), nnz, n, b, a,
+                                lower_only != 0, idx, code);
+  else
+    *count = bta::pattern_codes(static_cast<const int64_t*>(rows), static_cast<const int64_t*>(cols), nnz, n, b, a,
+                                lower_only != 0, idx, code);
   return 0;
 }
 

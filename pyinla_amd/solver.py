@@ -85,6 +85,7 @@ class SerinvSolver:
         self._ws = ws
         self._ld_out = torch.zeros(1, **f64)
         self._scatter_cache = {}
+        self._scatter_last = None  # (sparsity, rows, cols, map) of the last scatter
         self.total_bytes = 0
         self.t_cholesky = 0.0
         self.t_solve = 0.0
@@ -301,43 +302,24 @@ class SerinvSolver:
         (n, i) and the tip.  lower_only keeps i >= j only (the gather of
         structured_solver.py:470-538 works on tril(A)).
         """
-        from .st_model import bta_codes
         n, b = self.n_diag_blocks, self.diagonal_blocksize
         a = self.arrowhead_blocksize if sparsity == "bta" else 0
-        nb_ = n * b
-        rows = np.asarray(rows, dtype=np.int64)
-        cols = np.asarray(cols, dtype=np.int64)
-        st_r, st_c = rows < nb_, cols < nb_
-        bi = np.where(st_r, rows // b, n)
-        bj = np.where(st_c, cols // b, n)
-        keepD = st_r & st_c & (bi == bj)
-        keepL = st_r & st_c & (bi == bj + 1)
-        keep = keepD | keepL
-        if a > 0:
-            keep |= (~st_r) & (rows < nb_ + a) & ((cols < nb_) | (cols < nb_ + a))
-        if lower_only:
-            keep &= rows >= cols
-        idx = np.nonzero(keep)[0]
-        r, c = rows[idx], cols[idx]
-        # entries of the upper triangle of a diagonal block are stored as they
-        # are (the blocks hold both triangles, as in the reference)
-        upper = (r < c)
-        codes = np.empty(len(idx), dtype=np.uint64)
-        if (~upper).any():
-            codes[~upper] = bta_codes(r[~upper], c[~upper], n, b, a)
-        if upper.any():
-            ru, cu = r[upper], c[upper]
-            tip = (ru >= nb_)
-            cd = np.empty(len(ru), dtype=np.uint64)
-            if (~tip).any():  # inside a diagonal block: offset of (row, col) within D
-                blk = ru[~tip] // b
-                off = blk * b * b + (ru[~tip] % b) * b + (cu[~tip] % b)
-                cd[~tip] = off.astype(np.uint64)
-            if tip.any():
-                off = (ru[tip] - nb_) * a + (cu[tip] - nb_)
-                cd[tip] = (np.uint64(3) << np.uint64(60)) | off.astype(np.uint64)
-            codes[upper] = cd
-        return idx, codes
+        rows, cols = self._index_pair(rows, cols)
+        idx = np.empty(len(rows), dtype=np.int64)
+        codes = np.empty(len(rows), dtype=np.uint64)
+        count = C.c_int64()
+        _lib.check(self.lib.bta_pattern_codes(C.c_void_p(rows.ctypes.data), C.c_void_p(cols.ctypes.data),
+                                              rows.itemsize, len(rows), n, b, a, int(lower_only),
+                                              C.c_void_p(idx.ctypes.data), C.c_void_p(codes.ctypes.data),
+                                              C.byref(count)), "bta_pattern_codes")
+        return idx[:count.value], codes[:count.value]
+
+    @staticmethod
+    def _index_pair(rows, cols):
+        """Contiguous index arrays of one 4- or 8-byte integer type."""
+        rows, cols = np.asarray(rows), np.asarray(cols)
+        dt = np.int32 if rows.dtype == np.int32 and cols.dtype == np.int32 else np.int64
+        return np.ascontiguousarray(rows, dtype=dt), np.ascontiguousarray(cols, dtype=dt)
 
     @staticmethod
     def _pattern_key(rows, cols) -> bytes:
@@ -363,13 +345,22 @@ class SerinvSolver:
         else:
             coo = sps.coo_matrix(A)
             rows, cols, data = coo.row, coo.col, np.asarray(coo.data, dtype=np.float64)
-        key = (sparsity, len(data), self._pattern_key(rows, cols))
-        ent = self._scatter_cache.get(key)
-        if ent is None:
-            idx, codes = self._pattern_codes(rows, cols, sparsity, lower_only=False)
-            ent = (torch.from_numpy(idx.astype(np.int32)).to(self.device),
-                   torch.from_numpy(codes.view(np.int64)).to(self.device), len(idx))
-            self._scatter_cache[key] = ent
+        rows, cols = self._index_pair(rows, cols)
+        last = self._scatter_last
+        if last is not None and last[0] == sparsity and np.array_equal(last[1], rows) and \
+                np.array_equal(last[2], cols):
+            # the pattern of the call before, compared index by index: the
+            # digest of 350 k int64 pairs takes 4.6 ms, this 0.5
+            ent = last[3]
+        else:
+            key = (sparsity, len(data), self._pattern_key(rows, cols))
+            ent = self._scatter_cache.get(key)
+            if ent is None:
+                idx, codes = self._pattern_codes(rows, cols, sparsity, lower_only=False)
+                ent = (torch.from_numpy(idx.astype(np.int32)).to(self.device),
+                       torch.from_numpy(codes.view(np.int64)).to(self.device), len(idx))
+                self._scatter_cache[key] = ent
+            self._scatter_last = (sparsity, rows.copy(), cols.copy(), ent)
         src_idx, codes, count = ent
         for t in (self.A_diagonal_blocks, self.A_lower_diagonal_blocks, self.A_arrow_bottom_blocks,
                   self.A_arrow_tip_block):
