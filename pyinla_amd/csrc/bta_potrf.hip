@@ -21,7 +21,7 @@
 
 #include "bta_internal.h"
 #include "../../include/pyinla_bta.h"
-#include "bta_tile_chol.h"
+#include "bta_blocks16.h"
 
 namespace bta {
 
@@ -244,6 +244,128 @@ __global__ void k_begin_batch(const ProbDesc* probs, int nprob) {
     probs[q].info[0] = kInfoNone;
     probs[q].err[0] = 0;
   }
+}
+
+// ------------------------------------------------ one tile per block, b <= 64
+//
+// The whole factorization as one workgroup: a block is a single tile, so the
+// chain D_i -> L_i, B_i -> D_{i+1} has no parallel work for a second CU, and two
+// launches per block (k_panel_step and the update) spent more on the launches
+// and on passing the tile through memory than on the arithmetic.  Everything a
+// block hands to the next one stays in LDS or registers; the next block's
+// operands are loaded while this one is factored, and only the 16-wide block
+// columns that b has are factored.  Bound by the chain of pivots.  Measured on
+// MI355X, us per block (a = 6), against the two launches: b = 16 8.0 / 24.8, b = 40
+// 15.3 / 26.6, b = 64 18.2 / 26.3.
+struct ChainArgs {
+  double *D, *L, *B, *T;
+  double* Winv;     // n inverse tiles
+  double* logpart;  // n partial log sums
+  unsigned long long* info;
+  int n, b, a;
+};
+
+__global__ void __launch_bounds__(BTA_THREADS, 1) k_chain64(ChainArgs p) {
+  __shared__ double s[64 * BTA_LDS_LD];  // D_i, then its factor
+  __shared__ double w[64 * BTA_LDS_LD];  // the factor's inverse
+  __shared__ double x[64 * BTA_LDS_LD];  // L_i
+  __shared__ double y[64 * BTA_LDS_LD];  // B_i
+  const int n = p.n, b = p.b, a = p.a, nb = (b + 15) / 16, na = (a + 15) / 16;
+  const int64_t bb = (int64_t)b * b, ab = (int64_t)a * b;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // The 16x16 blocks of each product, dealt over the waves so that the four
+  // come out even: L_i = X W^T takes a block row per wave (10 of 16 products),
+  // D_{i+1} its lower triangle (3, 3, 2, 2), then the arrow's.
+  Blocks<4> xb, yb, bn;
+  Blocks<3> d, t;
+  xb.n = wv < nb ? nb : 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    xb.row[u] = 16 * wv;
+    xb.col[u] = 16 * u;
+  }
+  d.deal(nb, nb, true, 0);
+  yb.deal(na, nb, false, 3);
+  bn.deal(na, nb, false, 2);
+  t.deal(na, na, true, 2);
+  lds_load_tile(s, p.D, b, b, b);
+  if (a > 0) {
+    lds_load_tile(y, p.B, b, a, b);
+    t.load(p.T, a, a, a);
+  }
+  __syncthreads();
+  for (int i = 0; i < n; ++i) {
+    const bool next = i < n - 1;
+    double* Di = p.D + i * bb;
+    double* Li = p.L + i * bb;
+    double* Bi = p.B + i * ab;
+    TilePrefetch pl;
+    if (next) {
+      pl.load(Li, b, 0, b, b);
+      d.load(Di + bb, b, b, b);
+      if (a > 0) bn.load(Bi + ab, b, a, b);
+    }
+    if (b < 64) {
+      tile_chol_pad(s, w, b);
+      lds_barrier();
+    }
+    tile_chol_blocks<false>(s, w, b, [] {}, nb);
+    const double lii = s[lane * BTA_LDS_LD + lane];
+    if (next) pl.store(x, 0);
+    for (int r = wv; r < 64; r += 4) {
+      if (r < b && lane < b) Di[(int64_t)r * b + lane] = s[r * BTA_LDS_LD + lane];
+      p.Winv[(int64_t)i * 4096 + r * 64 + lane] = w[r * BTA_LDS_LD + lane];
+    }
+    lds_barrier();
+    xb.zero();
+    yb.zero();
+#pragma unroll
+    for (int k = 0; k < 64; k += 16) {
+      if (k >= b) break;
+      if (next) xb.product<false, 0, 0, true>(x, w, k);
+      yb.product<false, 0, 0, true>(y, w, k);
+    }
+    lds_barrier();
+    if (next) {
+      xb.to_lds(x);
+      xb.store(Li, b, b, b);
+    }
+    if (a > 0) {
+      yb.to_lds(y);
+      yb.store(Bi, b, a, b);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < 64; k += 16) {
+      if (k >= b) break;
+      if (next) {
+        d.product<true, 0, 0>(x, x, k);
+        bn.product<true, 0, 0>(y, x, k);
+      }
+      t.product<true, 0, 0>(y, y, k);
+    }
+    if (wv == 3) {
+      const TileCholResult res = tile_log_pivots(lii, b);
+      if (lane == 0) {
+        p.logpart[i] = res.logsum;
+        if (res.fail >= 0) atomicMin(p.info, (unsigned long long)((long long)i * b + res.fail));
+      }
+    }
+    lds_barrier();
+    if (next) {
+      d.to_lds(s);
+      if (a > 0) bn.to_lds(y);
+    }
+    lds_barrier();
+  }
+#pragma unroll
+  for (int u = 0; u < 3; ++u)
+    if (u < t.n)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = t.row[u] + 4 * q + (lane >> 4), c = t.col[u] + (lane & 15);
+        if (r < a && c <= r) p.T[(int64_t)r * a + c] = t.v[u][q];
+      }
 }
 
 // ------------------------------------------------------- block update GEMMs
@@ -543,7 +665,13 @@ int potrf_enqueue(Workspace& ws, double* D, double* L, double* B, double* T, int
   const bool flow = use_flow(ws, b) && ws.flow && ws.flow->nT == nT && ws.flow_sched && ws.flow_sched->nTa == nTa;
   if (use_flow(ws, b) && !flow) return (int)hipErrorNotReady;  // potrf_prepare not run for this shape
   hipLaunchKernelGGL(k_begin_call, dim3(1), dim3(64), 0, st, ws.epoch, ws.info, ws.err);
-  for (int i = 0; i < n; ++i) {
+  const bool chain = b <= 64 && a <= 64 && ws.panel_mode == 0 && !use_plan;
+  if (chain) {
+    TimedScope ts(ws, KC_PANEL, st);
+    hipLaunchKernelGGL(k_chain64, dim3(1), dim3(BTA_THREADS), 0, st,
+                       ChainArgs{D, L, B, T, ws.winv, ws.logpart, ws.info, n, b, a});
+  }
+  for (int i = 0; i < n && !chain; ++i) {
     PanelArgs p;
     p.D = D + (int64_t)i * b * b;
     p.L = (i < n - 1) ? L + (int64_t)i * b * b : nullptr;

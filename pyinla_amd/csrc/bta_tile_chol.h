@@ -68,9 +68,11 @@ __device__ __forceinline__ void store16_lower(double* __restrict__ C, int r0, in
   }
 }
 
-// acc +/-= X(rx.., kx..) * op(Y): NT form (ty == 0: Y rows ry.., K cols ky..),
-// or NN form (ty == 1: Y rows ky.. (K), cols ry..), K = 16, LDS stride BTA_LDS_LD.
-template <bool NEG, int TY>
+// acc +/-= op(X) * op(Y), K = 16, LDS stride BTA_LDS_LD.  X rows rx.., K cols
+// kx.. (TX == 0) or its transpose, rows kx.. (K), cols rx.. (TX == 1); Y in NT
+// form (TY == 0: rows ry.., K cols ky..) or NN form (TY == 1: rows ky.. (K),
+// cols ry..).
+template <bool NEG, int TY, int TX = 0>
 __device__ __forceinline__ f64x4 mma16x16(const double* __restrict__ X, int rx, int kx, const double* __restrict__ Y,
                                           int ry, int ky, f64x4 acc) {
   const int lane = threadIdx.x & 63;
@@ -78,7 +80,7 @@ __device__ __forceinline__ f64x4 mma16x16(const double* __restrict__ X, int rx, 
   double a[4], b[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    a[k] = X[(rx + li) * BTA_LDS_LD + kx + 4 * k + lk];
+    a[k] = TX == 0 ? X[(rx + li) * BTA_LDS_LD + kx + 4 * k + lk] : X[(kx + 4 * k + lk) * BTA_LDS_LD + rx + li];
     b[k] = TY == 0 ? Y[(ry + li) * BTA_LDS_LD + ky + 4 * k + lk] : Y[(ky + 4 * k + lk) * BTA_LDS_LD + ry + li];
   }
 #pragma unroll
@@ -215,13 +217,15 @@ __device__ __forceinline__ void clear_upper_blocks(double* __restrict__ s, doubl
 
 // The block columns of a tile in LDS; with FIRST the first one's diagonal block
 // is already factored (L_00 in s, E_00 in w, a full tile's upper blocks clear).
-// `spare` is run by wave 3 beside the last 16x16 factorization.
+// `spare` is run by wave 3 beside the last 16x16 factorization.  nblk: block
+// columns to factor (a padded tile's last ones are the identity already).
 template <bool FIRST, class F>
-__device__ __forceinline__ void tile_chol_blocks(double* __restrict__ s, double* __restrict__ w, int mv, F&& spare) {
+__device__ __forceinline__ void tile_chol_blocks(double* __restrict__ s, double* __restrict__ w, int mv, F&& spare,
+                                                 int nblk = 4) {
   const int tid = threadIdx.x;
   const int wv = tid >> 6;
 #pragma unroll 1
-  for (int jb = 0; jb < 4; ++jb) {
+  for (int jb = 0; jb < nblk; ++jb) {
     const int r0 = 16 * jb;
     if (!FIRST || jb > 0) {
       // ---- phase 1
@@ -234,7 +238,7 @@ __device__ __forceinline__ void tile_chol_blocks(double* __restrict__ s, double*
         if (mv == 64) clear_upper_blocks(s, w, tid - 64, BTA_THREADS - 64);
       } else {
         // trailing tiles of block column jb-1 other than (jb, jb), then the T_jk
-        const int nr = 4 - jb, nl = nr * (nr + 1) / 2 - 1;
+        const int nr = nblk - jb, nl = nr * (nr + 1) / 2 - 1;
         for (int t = wv - 1; t < nl + jb; t += 3) {
           if (t < nl) {
             int rr = 0, cc = t + 1;  // lower-triangle tile t+1 of the trailing block, row-major
@@ -254,21 +258,21 @@ __device__ __forceinline__ void tile_chol_blocks(double* __restrict__ s, double*
             store16(w, r0, 16 * k, acc);
           }
         }
-        if (jb == 3 && wv == 3) spare();
+        if (jb == nblk - 1 && wv == 3) spare();
       }
       lds_barrier();
     }
-    // ---- phase 2: product q < 3 - jb is L_(jb+1+q),jb, the others E_jb,(q - (3 - jb))
+    // ---- phase 2: product q < nd is L_(jb+1+q),jb, the others E_jb,(q - nd)
     {
-      const int q = (jb < 3) ? (wv <= 2 ? wv : -1) : wv - 1;
-      if (q >= 0) {
+      const int nd = nblk - 1 - jb, q = nd > 0 ? wv : wv - 1;
+      if (q >= 0 && q < nblk - 1) {
         f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
-        if (q < 3 - jb) {
+        if (q < nd) {
           const int ib = jb + 1 + q;
           acc = mma16x16<false, 0>(s, 16 * ib, r0, w, r0, r0, acc);  // A_ib,jb E_jj^T
           store16(s, 16 * ib, r0, acc);
         } else {
-          const int k = q - (3 - jb);
+          const int k = q - nd;
           acc = mma16x16<true, 1>(w, r0, r0, w, 16 * k, r0, acc);    // -E_jj T_jk
           store16(w, r0, 16 * k, acc);
         }
@@ -278,12 +282,13 @@ __device__ __forceinline__ void tile_chol_blocks(double* __restrict__ s, double*
   }
 }
 
-// Identity outside the valid block, zero strict upper triangle, E = 0.
+// Identity outside the valid block, in s and E alike, zero strict upper
+// triangle, E = 0 inside.
 __device__ __forceinline__ void tile_chol_pad(double* __restrict__ s, double* __restrict__ w, int mv) {
   for (int e = threadIdx.x; e < 64 * 64; e += BTA_THREADS) {
     const int i = e >> 6, j = e & 63;
     if (i >= mv || j >= mv || j > i) s[i * BTA_LDS_LD + j] = (i == j) ? 1.0 : 0.0;
-    w[i * BTA_LDS_LD + j] = 0.0;
+    w[i * BTA_LDS_LD + j] = (i == j && i >= mv) ? 1.0 : 0.0;
   }
 }
 
