@@ -106,6 +106,7 @@ struct PotriPlan {
     double beta;      // 1 when the arrow term is already in C
   };
   DevPlan grouped;    // every product in the grouped kernel
+  bool chain = false;  // the recurrence runs as k_chain64_selinv after them
   DevPlan with_blas;  // grouped launches of the variant with dgemm calls
   std::vector<BlasGemm> gemms;
   std::vector<int> order;
