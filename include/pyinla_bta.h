@@ -172,8 +172,8 @@ int bta_logdet(bta_ws_t ws, const double* D, const double* T, int n, int b, int 
 #define BTA_OPT_FLOW_HELPERS 4
 #define BTA_OPT_FLOW_DELTA 5
 /* Batched factorization in the persistent form: problems factored
- * concurrently per wave (taken from the first problem's workspace; 0 = 6,
- * at most 8). */
+ * concurrently per wave (taken from the first problem's workspace; 0 =
+ * automatic, at most 20). */
 #define BTA_OPT_BATCH_LANES 6
 /* Selected inversion: 1 (default) = for b > 1600 the b x b x b products
  * Sigma_{i+1,i} = -Sigma_{i+1,i+1} G_i as rocBLAS dgemm calls on the caller's

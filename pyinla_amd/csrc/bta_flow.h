@@ -128,8 +128,9 @@ struct FlowArgs {
 
 // Entries of one batched launch, passed by value: pointers in kernel
 // arguments are known to the compiler to be global (read from a table in
-// memory they would be generic and every access a FLAT one).
-#define FLOW_BATCH_MAX 8
+// memory they would be generic and every access a FLAT one).  20 entries are
+// 3.8 KB of the 4 KB of kernel arguments.
+#define FLOW_BATCH_MAX 20
 // Workgroup layout of a batched launch.  iso == 0: entry q owns workgroups
 // [begin[q], begin[q+1]), its chain first.  iso == 1 (two workgroups per CU,
 // workgroup p sharing its CU with workgroup p + cus): the chains are

@@ -1218,6 +1218,7 @@ __global__ void __launch_bounds__(BTA_THREADS, 2) k_panel_flow_batched(FlowBatch
     if (wg < fb.nent) pos = -1;                         // chain of entry wg
     else pos = wg < fb.cus ? wg - fb.nent : wg - 2 * fb.nent;
   }
+  if (pos >= fb.begin[fb.nent]) return;
   int lo = 0, local = 0;
   if (pos < 0) {
     lo = wg;

@@ -168,7 +168,7 @@ struct Workspace {
   int flow_near = 16;    // near pool = helpers / flow_near (see flow_near_pool)
   int flow_fold = 0;     // block update: 0 = automatic, 1 = in the persistent panel, 2 = a grouped GEMM after it
   int gemm_variant = 0;  // grouped GEMM: 0 = chosen by pick_kernel, 1 = two LDS buffers
-  int batch_lanes = 0;   // problems per wave of a batched factorization (0 = 6)
+  int batch_lanes = 0;   // problems per wave of a batched factorization (0 = automatic)
   // persistent-panel exchange buffers, sized for the workspace's arrowhead
   // (allocated by bta_ws_create when the flow panel can run)
   std::unique_ptr<FlowPlan> flow;
@@ -254,7 +254,7 @@ struct BatchPlan {
   BatchPlan(const BatchPlan&) = delete;
   BatchPlan& operator=(const BatchPlan&) = delete;
   ~BatchPlan();
-  // lanes: problems factored concurrently in the persistent form (0 = 6,
+  // lanes: problems factored concurrently in the persistent form (0 = automatic,
   // at most FLOW_BATCH_MAX)
   int build(const std::vector<ProbDesc>& ps, int panel_mode, int lanes, int delta, int near_div, int device);
   int enqueue(hipStream_t st) const;

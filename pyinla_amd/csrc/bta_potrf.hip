@@ -733,23 +733,101 @@ BatchPlan::~BatchPlan() {
   if (d_ent) hipFree(d_ent);
 }
 
+// Helpers of the problems of one launch, `each` on average.  The launch takes
+// as long as its slowest problem, so they go by the work of a problem's block,
+// nT^3 tile products, beyond two per tile column, which is what keeps a small
+// problem bound by its chain.  Equal problems get equal shares.  Measured on
+// MI355X, six problems of b = 256 .. 2048, 8 .. 40 blocks: 17.9 ms with equal
+// shares (1750 us for a step with b = 2048), 11.0 by work.
+static std::vector<int> helper_shares(const std::vector<int>& nT, int each) {
+  const int np = (int)nT.size(), total = each * np;
+  std::vector<int> h(np);
+  double work = 0.0;
+  int given = 0;
+  for (int q = 0; q < np; ++q) {
+    h[q] = std::min(each, 2 * nT[q]);
+    given += h[q];
+    work += (double)nT[q] * nT[q] * nT[q];
+  }
+  const int rest = total - given;
+  for (int q = 0; q < np; ++q)
+    h[q] = std::min(1023, h[q] + (int)(rest * ((double)nT[q] * nT[q] * nT[q] / work) + 1e-6));
+  return h;
+}
+
+// A block step in us, from lone and batched launches on MI355X: the chain takes
+// 15.2 us per tile column, a block 3.3 nT^3 us of one helper that has its CU to
+// itself and 4.5 of one that shares it.
+static double step_work(const std::vector<int>& nT) {
+  double w = 0.0;
+  for (const int t : nT) w += (double)t * t * t;
+  return w;
+}
+static double step_chain(const std::vector<int>& nT) { return 15.2 * *std::max_element(nT.begin(), nT.end()); }
+// One workgroup per CU is enough to keep the longest chain the bound (a second
+// one on some CUs makes those helpers late: b = 1600 with b = 100 4.3 ms per 10
+// blocks, 3.9 with one per CU).
+static bool step_fits_one(const std::vector<int>& nT, int cus) {
+  const int np = (int)nT.size(), h = cus / np - 1;
+  return h >= 1 && 3.3 * step_work(nT) <= step_chain(nT) * h * np;
+}
+static double step_time(const std::vector<int>& nT, int cus, int cap) {
+  if (step_fits_one(nT, cus)) return step_chain(nT);
+  return std::max(step_chain(nT), 4.5 * step_work(nT) / std::max(1, cap - 2 * (int)nT.size()));
+}
+
+// Problems per wave: the number that the estimate above says is fastest, by the
+// steps of all waves and 10 us per launch.  Chains side by side cost nothing
+// until the helpers are the bound.  Finite-difference stencil of 18 problems,
+// nt = 16, in ms as waves of 6, 9, 18: b = 120 5.5, 4.9, 4.4; b = 480 11.0, 9.8,
+// 8.4; b = 840 21.7, 20.0, 21.6.
+static int pick_lanes(const std::vector<ProbDesc>& ps, const std::vector<int>& order, int cus, int cap) {
+  const int np = (int)ps.size();
+  int best = 1;
+  double best_t = 0.0;
+  for (int nl = 1; nl <= std::min(np, FLOW_BATCH_MAX) && cap / nl - 1 >= 1; ++nl) {
+    double t = 0.0;
+    for (int w0 = 0; w0 < np; w0 += nl)
+      for (int i = 0; i < ps[order[w0]].n;) {  // longest first
+        std::vector<int> nts;
+        int until = 1 << 30;
+        for (int q = w0; q < std::min(np, w0 + nl); ++q)
+          if (i < ps[order[q]].n) {
+            nts.push_back(ps[order[q]].nT);
+            until = std::min(until, ps[order[q]].n);
+          }
+        t += (until - i) * (step_time(nts, cus, cap) + 10.0);
+        i = until;
+      }
+    if (nl == 1 || t < best_t) {
+      best = nl;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
 int BatchPlan::build(const std::vector<ProbDesc>& ps, int panel_mode, int lanes, int delta, int near_div,
                      int device) {
   probs = ps;
   // Persistent dataflow form when every problem has more than one tile column
-  // (or when asked for): each problem gets a chain and an equal share of the
-  // device's resident workgroups as helpers, all in one launch per block step.
+  // (or when asked for): each problem gets a chain and a share of the device's
+  // resident workgroups as helpers, all in one launch per block step.
   bool all_wide = true;
   for (const auto& d : ps) all_wide = all_wide && d.b > 64;
   flow = (panel_mode == 2) || (panel_mode == 0 && all_wide);
   if (flow) {
-    // helpers per problem: the device's resident capacity split evenly over
-    // the problems still active at each block step
+    // helpers per problem: the device's resident capacity split over the
+    // problems still active at each block step
     const int cap = flow_capacity(device);
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 0;
     const int np = (int)ps.size();
-    const int nl = std::min(lanes > 0 ? std::min(lanes, np) : std::min(np, 6), FLOW_BATCH_MAX);
+    // problems run longest first, in waves of at most nl
+    std::vector<int> order(np);
+    for (int q = 0; q < np; ++q) order[q] = q;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ps[x].n > ps[y].n; });
+    const int nl = std::min(lanes > 0 ? std::min(lanes, np) : pick_lanes(ps, order, cus, cap), FLOW_BATCH_MAX);
     if (cap / nl - 1 < 1) {
       flow = false;  // too many problems to give each a resident chain + helper
     } else {
@@ -772,12 +850,8 @@ int BatchPlan::build(const std::vector<ProbDesc>& ps, int panel_mode, int lanes,
         owned.back()->spin_ticks = flow_spin_ticks(device, 20.0);
         fplans.push_back(owned.back().get());
       }
-      // Problems run in waves of at most `lanes` (longest first), so that each
-      // chain gets enough helpers; within a wave every launch covers the
-      // wave's problems that still have block step i.
-      std::vector<int> order(np);
-      for (int q = 0; q < np; ++q) order[q] = q;
-      std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ps[x].n > ps[y].n; });
+      // Within a wave every launch covers the wave's problems that still have
+      // block step i.
       for (int w0 = 0; w0 < np; w0 += nl) {
         const int w1 = std::min(np, w0 + nl);
         int wmax = 0;
@@ -785,32 +859,43 @@ int BatchPlan::build(const std::vector<ProbDesc>& ps, int panel_mode, int lanes,
         for (int i = 0; i < wmax; ++i) {
           int nact = 0;
           for (int t = w0; t < w1; ++t) nact += (i < ps[order[t]].n) ? 1 : 0;
+          std::vector<int> nts;
+          for (int t = w0; t < w1; ++t)
+            if (i < ps[order[t]].n) nts.push_back(ps[order[t]].nT);
+          const int h_one = cus / nact - 1, h_iso = (cap - 2 * nact) / nact;
+          const bool one = step_fits_one(nts, cus);
+          const bool two = !one && cus > 0 && cap == 2 * cus && h_iso >= 1;
+          const std::vector<int> shares = helper_shares(nts, one ? h_one : (two ? h_iso : cap / nact - 1));
+          int sum = 0;
+          for (const int h : shares) sum += h;
           // two workgroups per CU: each chain gets a CU of its own (its
           // partner slot idle), measured on MI355X to shorten the chain's
-          // steps as much as a co-resident helper had lengthened them
-          const int h_iso = (cap - 2 * nact) / nact;
-          const bool iso = cus > 0 && cap == 2 * cus && h_iso >= 1 && nact * (2 + h_iso) >= cus + nact;
-          const int helpers = std::min(1023, iso ? h_iso : cap / nact - 1);
+          // steps as much as a co-resident helper had lengthened them.  The
+          // idle slots are workgroups cus .. cus + nact - 1: the launch has to
+          // reach past them.
+          const bool iso = two && sum + 2 * nact >= cus + nact;
           FLaunch L;
           L.fb.nent = 0;
           L.fb.iso = iso ? 1 : 0;
           L.fb.cus = cus;
-          int total = 0;
+          int total = 0, before = 0;
           for (int t = w0; t < w1; ++t) {
             const int q = order[t];
             const ProbDesc& d = ps[q];
             if (i >= d.n) continue;
+            const int helpers = shares[L.fb.nent];
             const FlowSched* sc = nullptr;
             const int rc = fplans[q]->sched(d.a > 0 ? d.nTa : 0, helpers, delta, near_div, 1, &sc);
             if (rc) return rc;
             L.fb.e[L.fb.nent] = flow_args(*fplans[q], *sc, d.D, d.L, d.B, d.T, d.winv, d.logpart, d.epoch,
                                           d.info, d.err, i, d.n, d.b, d.a);
             const int j = L.fb.nent;
-            L.fb.begin[j] = iso ? j * helpers : total;  // iso: helper numbers
+            L.fb.begin[j] = iso ? before : total;  // iso: helper numbers
             L.fb.nent = j + 1;
             total += 1 + helpers;
+            before += helpers;
           }
-          L.fb.begin[L.fb.nent] = iso ? L.fb.nent * helpers : total;
+          L.fb.begin[L.fb.nent] = iso ? before : total;
           L.total = iso ? total + L.fb.nent : total;  // + the chains' idle partners
           flaunches.push_back(L);
         }
