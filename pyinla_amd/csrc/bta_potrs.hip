@@ -24,7 +24,7 @@
 //   b = 800           3.0 / 3.3     (8.6 / 11.1)
 //   b = 1600          5.2 / 6.1     (11.3 / 13.7) its bytes at 5 TB/s: 3.1
 //   b = 4500          27 / 37       (37 / 37)     its bytes at 5 TB/s: 24
-//   b = 800, 16 right-hand sides    14 / 17       (78 / 55)
+//   b = 800, 16 right-hand sides    7 / 9         (78 / 55)
 #include <algorithm>
 
 #include "bta_internal.h"
@@ -57,7 +57,16 @@ struct SweepArgs {
   unsigned long long spin_ticks;
   int n, b, a, ldx, nr;        // nr <= R right-hand sides
   int parts;                   // work items per product
-  int seats;                   // workgroups launched
+  int seats;                   // workgroups per group of R right-hand sides
+  int64_t gstride;             // doubles from one group's scratch to the next's
+
+  // Groups of R columns run side by side: the arguments of group g.
+  __device__ __forceinline__ void enter_group(int R, int g) {
+    X += (int64_t)g * R;
+    vec += g * gstride;
+    claims += g * gstride * (int64_t)(sizeof(double) / sizeof(unsigned));
+    nr = min(R, nr - g * R);
+  }
 };
 
 // Length of a hand-over vector: whole 128-byte lines.
@@ -328,10 +337,10 @@ struct SweepWait {
 // see the vector only after them).  With several right-hand sides, whose vectors
 // are larger, all waves do.
 template <int R, int U, bool T, int NP>
-__device__ __forceinline__ void sweep_poller(const SweepArgs& p, SweepLds<R, U, T>& l, int stages) {
+__device__ __forceinline__ void sweep_poller(const SweepArgs& p, SweepLds<R, U, T>& l, int stages, int own) {
   using Lds = SweepLds<R, U, T>;
   const int t = (int)threadIdx.x - kSweepThreads;
-  SweepWalk walk(p, stages, blockIdx.x);
+  SweepWalk walk(p, stages, own);
   unsigned patience = kPatience;
   unsigned long long t1 = 0;
   int turn = 0;
@@ -368,13 +377,13 @@ __device__ __forceinline__ void sweep_poller(const SweepArgs& p, SweepLds<R, U, 
 // Waves that multiply: 8 of them, each with up to U 16-byte loads of the
 // item's matrix in flight while the others wait.
 template <int R, int U, bool T, int NP>
-__device__ __forceinline__ void sweep_worker(const SweepArgs& p, SweepLds<R, U, T>& l, int stages) {
+__device__ __forceinline__ void sweep_worker(const SweepArgs& p, SweepLds<R, U, T>& l, int stages, int own) {
   using Lds = SweepLds<R, U, T>;
   constexpr int RK = Lds::RK, LV = Lds::LV, NO = Lds::NO, NA = T ? 2 * R : R;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = p.b, a = p.a;
   const int64_t half = vec_len(b, R), vlen = T ? 2 * half : half;
-  SweepWalk walk(p, stages, blockIdx.x);
+  SweepWalk walk(p, stages, own);
   int turn = 0;
   auto settle = [&](int seat) { return sweep_settle(l, walk, turn, seat, false, [](int) { return 0; }); };
   do {
@@ -505,9 +514,11 @@ template <int R, int U, bool T, int NP>
 __global__ void __launch_bounds__(kSweepThreads + 64 * NP, 4) k_sweep(SweepArgs p) {
   __shared__ SweepLds<R, U, T> l;
   const int stages = 2 * p.n - ((T && p.a > 0) ? 0 : 1);
+  const int group = (int)blockIdx.x / p.seats, own = (int)blockIdx.x - group * p.seats;
+  p.enter_group(R, group);
   if (threadIdx.x == 0) {
-    l.dead = claim_seat(p.claims + blockIdx.x) != 0;
-    l.seat[0] = blockIdx.x;
+    l.dead = claim_seat(p.claims + own) != 0;
+    l.seat[0] = own;
     l.victim[0] = l.victim[1] = kSeats;
   }
   if constexpr (T)
@@ -515,8 +526,8 @@ __global__ void __launch_bounds__(kSweepThreads + 64 * NP, 4) k_sweep(SweepArgs 
       l.xa[e] = (e % R < p.nr) ? p.X[((int64_t)p.n * p.b + e / R) * p.ldx + e % R] : 0.0;
   __syncthreads();
   if (__builtin_amdgcn_readfirstlane(l.dead)) return;
-  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= kSweepThreads / 64) sweep_poller<R, U, T, NP>(p, l, stages);
-  else sweep_worker<R, U, T, NP>(p, l, stages);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= kSweepThreads / 64) sweep_poller<R, U, T, NP>(p, l, stages, own);
+  else sweep_worker<R, U, T, NP>(p, l, stages, own);
 }
 
 // Before a sweep: the hand-over vectors (vector 0: the first block of the
@@ -527,7 +538,8 @@ __global__ void __launch_bounds__(kSweepThreads + 64 * NP, 4) k_sweep(SweepArgs 
 __global__ void __launch_bounds__(BTA_THREADS) k_sweep_init(SweepArgs p, const double* x0, int R, int pieces,
                                                            int64_t vectors, int64_t nclaims, double* Xtip,
                                                            const double* tinv, int tip) {
-  if (blockIdx.x == 0) {
+  const int group = blockIdx.y;
+  if (blockIdx.x == 0 && group == 0) {
     const int a = p.a, per = tip > 0 ? BTA_THREADS / a : 1;
     for (int c0 = 0; c0 < tip; c0 += per) {
       const int q = threadIdx.x / per, rc = c0 + threadIdx.x % per;
@@ -540,6 +552,8 @@ __global__ void __launch_bounds__(BTA_THREADS) k_sweep_init(SweepArgs p, const d
       __syncthreads();
     }
   }
+  p.enter_group(R, group);
+  x0 += (int64_t)group * R;
   const int64_t len = (int64_t)p.b * R, pad = vec_len(p.b, R);
   const int64_t t0 = (int64_t)blockIdx.x * BTA_THREADS + threadIdx.x, stride = (int64_t)gridDim.x * BTA_THREADS;
   for (int64_t e = t0; e < vectors * pad; e += stride) {
@@ -553,6 +567,7 @@ __global__ void __launch_bounds__(BTA_THREADS) k_sweep_init(SweepArgs p, const d
 
 // After a backward sweep: X_i = sum of the two partial vectors of W_i's stage.
 __global__ void __launch_bounds__(BTA_THREADS) k_sweep_finish(SweepArgs p, int R) {
+  p.enter_group(R, blockIdx.y);
   const int64_t len = (int64_t)p.b * R, pad = vec_len(p.b, R), tot = p.n * len;
   const int first = p.a > 0 ? 0 : 1;
   for (int64_t e = (int64_t)blockIdx.x * BTA_THREADS + threadIdx.x; e < tot; e += (int64_t)gridDim.x * BTA_THREADS) {
@@ -775,8 +790,11 @@ __global__ void __launch_bounds__(BTA_THREADS) k_sweep_arrow(SweepArgs p, const 
   }
 }
 
+// Groups of R right-hand sides from column p.X on (p.nr in all), side by side
+// as far as `groups` scratches and the CUs go.  Returns the columns done.
 template <int R, int U, int NP>
-void sweep_group(Workspace& ws, SweepArgs p, const double* x0, double* Xtip, int tip, int trans, hipStream_t st) {
+int sweep_group(Workspace& ws, SweepArgs p, const double* x0, double* Xtip, int tip, int trans, int groups,
+                hipStream_t st) {
   p.parts = trans ? 2 * ((p.b + 15) / 16) : (p.b + 7) / 8;
   // one workgroup per CU; two where a product has more items than that (their
   // rounds of loads then overlap: b = 4500 27 / 37 us per product forward /
@@ -785,20 +803,26 @@ void sweep_group(Workspace& ws, SweepArgs p, const double* x0, double* Xtip, int
   p.seats = std::min(p.parts, std::min(R == 1 && U == 8 && p.b > 2048 ? 2 * ws.cus : ws.cus, kSeats));
   const int64_t products = 2 * (int64_t)p.n - ((trans && p.a > 0) ? 0 : 1), len = vec_len(p.b, R);
   const int64_t vectors = (products + 1) * (trans ? 2 : 1);
-  p.vec = ws.work;
-  p.claims = reinterpret_cast<unsigned*>(ws.work + vectors * len);
+  p.gstride = vectors * len + kSeats / 2;
+  groups = std::max(1, std::min({groups, (p.nr + R - 1) / R, ws.cus / p.seats}));
+  p.nr = std::min(p.nr, groups * R);
   auto grid = [](int64_t e, int cap) {
     return dim3((unsigned)std::min<int64_t>((e + BTA_THREADS - 1) / BTA_THREADS, cap));
   };
-  hipLaunchKernelGGL(k_sweep_init, grid(vectors * len, 1024), dim3(BTA_THREADS), 0, st, p, x0, R, trans ? 2 : 1,
-                     vectors, (int64_t)kSeats, Xtip, ws.tinv, tip);
-  const dim3 wgs(p.seats), th(kSweepThreads + 64 * NP);
+  p.vec = ws.work;
+  p.claims = reinterpret_cast<unsigned*>(ws.work + vectors * len);
+  const int columns = p.nr;
+  auto cover = [&](int64_t e) { return dim3(grid(e, 1024).x, groups); };
+  hipLaunchKernelGGL(k_sweep_init, cover(vectors * len), dim3(BTA_THREADS), 0, st, p, x0, R, trans ? 2 : 1, vectors,
+                     (int64_t)kSeats, Xtip, ws.tinv, tip);
+  const dim3 wgs(p.seats * groups), th(kSweepThreads + 64 * NP);
   if (trans) {
     hipLaunchKernelGGL((k_sweep<R, U, true, NP>), wgs, th, 0, st, p);
-    hipLaunchKernelGGL(k_sweep_finish, grid((int64_t)p.n * p.b * R, 1024), dim3(BTA_THREADS), 0, st, p, R);
+    hipLaunchKernelGGL(k_sweep_finish, cover((int64_t)p.n * p.b * R), dim3(BTA_THREADS), 0, st, p, R);
   } else {
     hipLaunchKernelGGL((k_sweep<R, U, false, NP>), wgs, th, 0, st, p);
   }
+  return columns;
 }
 
 template <int R, int K>
@@ -814,15 +838,25 @@ static size_t group_doubles(int n, int b, int R) {
   return (2 * (size_t)n + 1) * 2 * (size_t)vec_len(b, R) + kSeats / 2;
 }
 
-// Right-hand sides per pass (8, 4 or 1): as many as fit a scratch of 3 b^2
-// doubles, or 32 MB where that is more.
+// A scratch of 3 b^2 doubles, or 32 MB where that is more.
+static size_t sweep_room(int b) { return std::max(3 * (size_t)b * b, (size_t)1 << 22); }
+
+// Right-hand sides per group (8, 4 or 1): as many as fit the scratch.
 static int group_size(int n, int b) {
-  const size_t room = std::max(3 * (size_t)b * b, (size_t)1 << 22);
+  const size_t room = sweep_room(b);
   return group_doubles(n, b, 8) <= room ? 8 : (group_doubles(n, b, 4) <= room ? 4 : 1);
 }
 
+// Groups of that size that the scratch holds side by side: what fits as well, at
+// most 4.
+static int group_count(int n, int b) {
+  return (int)std::max<size_t>(1, std::min<size_t>(4, sweep_room(b) / group_doubles(n, b, group_size(n, b))));
+}
+
 // Scratch of the sweeps in doubles (0: swept by single workgroups).
-size_t sweep_doubles(int n, int b) { return b <= kSolo ? 0 : group_doubles(n, b, group_size(n, b)); }
+size_t sweep_doubles(int n, int b) {
+  return b <= kSolo ? 0 : group_count(n, b) * group_doubles(n, b, group_size(n, b));
+}
 
 int potrs_enqueue(Workspace& ws, const double* L, const double* B, int n, int b, int a, double* rhs, int nrhs,
                   int ldrhs, int trans, hipStream_t st) {
@@ -841,6 +875,7 @@ int potrs_enqueue(Workspace& ws, const double* L, const double* B, int n, int b,
   p.ldx = ldrhs;
   p.nr = nrhs;
   p.parts = p.seats = 0;
+  p.gstride = 0;
   double* Xtip = rhs + (int64_t)n * b * ldrhs;
   int tip = (trans && a > 0) ? nrhs : 0;
   TimedScope ts(ws, KC_GEMV, st);
@@ -851,20 +886,49 @@ int potrs_enqueue(Workspace& ws, const double* L, const double* B, int n, int b,
     if (nrhs == 1) sweep_solo<1, 8>(p, nrhs, trans, st);
     else sweep_solo<4, 8>(p, nrhs, trans, st);
   } else {
-    // groups of up to 8 right-hand sides share one pass over the factor
-    const int most = group_size(n, b);
+    // Groups of 1, 4 or 8 right-hand sides share one pass over the factor, as
+    // many groups side by side as the scratch and the CUs hold: the size whose
+    // passes take the least (one of 1, 4 and 8 is as 1 : 1.6 : 2.5).  Measured on
+    // MI355X, ms for 1, 4, 8, 16, 32 right-hand sides, in brackets with one
+    // group of 4 or 8 after the other:
+    //   n = 50, b = 92     0.37 0.37 0.38 0.41 0.79   (0.36 0.62 0.95 1.87 3.72)
+    //   n = 40, b = 300    0.32 0.34 0.61 0.64 0.99   (0.32 0.60 0.91 1.80 3.57)
+    //   n = 40, b = 800    0.50 0.77 0.78 1.24 2.51   (0.50 0.79 1.22 2.44 4.92)
     const double* x0 = rhs + (trans ? (int64_t)(n - 1) * b * ldrhs : 0);
+    const int room = std::max(1, ws.cus / std::min((b + 7) / 8, ws.cus));
+    auto slots = [&](int R) { return (int)std::min<size_t>(ws.work_doubles / group_doubles(n, b, R), room); };
+    const int size[3] = {1, 4, 8}, cols[3] = {std::max(1, slots(1)), 4 * slots(4), 8 * slots(8)};
+    const double pass[3] = {1.0, 1.6, 2.5};
+    auto passes_of_one_size = [&](int left) {  // the least time for the rest
+      double t = 0.0;
+      for (int q = 0; q < 3; ++q)
+        if (cols[q] > 0) {
+          const double x = pass[q] * ((left + cols[q] - 1) / cols[q]);
+          t = q == 0 ? x : std::min(t, x);
+        }
+      return t;
+    };
     for (int c0 = 0; c0 < nrhs;) {
-      const int R = std::min(most, nrhs - c0 == 1 ? 1 : (nrhs - c0 <= 4 ? 4 : 8));
+      int R = 1;
+      double best = 0.0;
+      for (int q = 0; q < 3; ++q) {
+        if (cols[q] == 0) continue;
+        const double t = pass[q] + passes_of_one_size(std::max(0, nrhs - c0 - cols[q]));
+        if (q == 0 || t < best) {
+          R = size[q];
+          best = t;
+        }
+      }
+      const int groups = slots(R);
       p.X = rhs + c0;
-      p.nr = std::min(R, nrhs - c0);
-      if (R == 1 && b <= 512) sweep_group<1, 4, 4>(ws, p, x0 + c0, Xtip, tip, trans, st);
-      else if (R == 1 && (b <= 1024 || b > 2048)) sweep_group<1, 8, 4>(ws, p, x0 + c0, Xtip, tip, trans, st);
-      else if (R == 1) sweep_group<1, 16, 4>(ws, p, x0 + c0, Xtip, tip, trans, st);
-      else if (R == 4) sweep_group<4, 8, 4>(ws, p, x0 + c0, Xtip, tip, trans, st);
-      else sweep_group<8, 8, 4>(ws, p, x0 + c0, Xtip, tip, trans, st);
+      p.nr = nrhs - c0;
+      const double* x = x0 + c0;
+      if (R == 1 && b <= 512) c0 += sweep_group<1, 4, 4>(ws, p, x, Xtip, tip, trans, groups, st);
+      else if (R == 1 && (b <= 1024 || b > 2048)) c0 += sweep_group<1, 8, 4>(ws, p, x, Xtip, tip, trans, groups, st);
+      else if (R == 1) c0 += sweep_group<1, 16, 4>(ws, p, x, Xtip, tip, trans, groups, st);
+      else if (R == 4) c0 += sweep_group<4, 8, 4>(ws, p, x, Xtip, tip, trans, groups, st);
+      else c0 += sweep_group<8, 8, 4>(ws, p, x, Xtip, tip, trans, groups, st);
       tip = 0;
-      c0 += p.nr;
     }
   }
   if (!trans && a > 0) {

@@ -126,3 +126,16 @@ def test_two_sweeps_share_the_device(cuda):
         ref = _oracle(kf, R[:, None].copy())[:, 0]
         assert np.abs(x.cpu().numpy() - ref).max() <= TOL * np.abs(ref).max()
         assert s.status()[0] == 0
+
+
+@pytest.mark.parametrize("n,b,a,nrhs", [(5, 65, 2, 33), (3, 130, 0, 17), (40, 200, 3, 25), (3, 520, 4, 23),
+                                        (2, 1030, 5, 16), (200, 70, 1, 32)])
+def test_groups_side_by_side(cuda, n, b, a, nrhs):
+    """Groups of 8 in one launch: 4 and fewer at a time, the last one ragged,
+    and the next launch's right behind."""
+    kf, s = _factored(n, b, a, seed=b + nrhs)
+    R = np.random.default_rng(b).normal(size=(n * b + a, nrhs))
+    ref = _oracle(kf, R)
+    for _ in range(2):
+        got = s.solve(torch.from_numpy(R.copy()).to(cuda), "bta" if a else "bt").cpu().numpy()
+        assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
