@@ -416,7 +416,7 @@ def main():
         roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                 "frac": ach / PEAK_FP64_TFLOPS, "traffic": None}
     roof["kernel"] = {0: "k_panel_flow" if flow else "k_panel_step", 1: "k_gemm_nt_sub", 2: "k_gemm_grouped",
-                      3: "k_gemv", 4: "rocblas_dgemm"}[dom]
+                      3: "k_sweep", 4: "rocblas_dgemm"}[dom]
     # HBM bytes per launch of that kernel from the committed rocprofv3 PMC
     # summary (FETCH_SIZE / WRITE_SIZE, scaled by a 1 GiB copy), if present
     tr_path = ROOT / "profiles" / "pmc_traffic.json"

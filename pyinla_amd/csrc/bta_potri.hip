@@ -262,10 +262,9 @@ int potri_build(Workspace& ws, PotriPlan& pp, double* D, double* L, double* B, d
   //   l2(i): Sigma_{i+1,i} = -Sigma_{i+1,i+1} G_i - Sigma_{n,i+1}^T Ga_i   (into L_i)
   //   l3(i): Sigma_ii     +=  - G_i^T Sigma_{i+1,i} - Ga_i^T Sigma_{n,i}  (into D_i)
   //          Sigma_{n,i-1} = -Sigma_{n,i} G_{i-1} - Sigma_T Ga_{i-1}     (into B_{i-1})
-  // Sigma_{n,i-1} needs only Sigma_{n,i}, so it rides in l3(i), whose
-  // lower-triangle tiles fill half of the resident slots, and l2 keeps its
-  // b x b tiles (one full wave at b = 2000).  Sigma_{n,n-1} = -Sigma_T Ga_{n-1}
-  // is l2(n-1).  Ga_i = B_i W_i was formed in l0, so B_{i-1} is free.
+  // Sigma_{n,i-1} needs only Sigma_{n,i}, so it rides in l3(i) instead of
+  // adding tiles to l2.  Sigma_{n,n-1} = -Sigma_T Ga_{n-1} is l2(n-1).  Ga_i =
+  // B_i W_i was formed in l0, so B_{i-1} is free.
   auto arrow_job = [&](int i) {  // Sigma_{n,i}
     double* Bi = B + (int64_t)i * a * b;
     GemmJob s2 = job(Bi, a, b, b, 0.0);
