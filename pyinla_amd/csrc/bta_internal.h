@@ -160,7 +160,7 @@ struct Workspace {
   // Output-tile edge per GEMM class: 0 = heuristic (pick_tile), 64 or 128.
   int tile_update = 0;   // block updates of the factorization
   int tile_grouped = 0;  // block inverses and selected inversion
-  // Panel factorization: 0 = automatic, 1 = one launch per tile column,
+  // Panel factorization: 0 = automatic (b <= 64: k_chain64), 1 = one launch per tile column,
   // 2 = persistent dataflow launch per block (bta_flow.hip).
   int panel_mode = 0;
   int flow_helpers = 0;  // 0 = automatic
