@@ -160,7 +160,8 @@ int bta_logdet(bta_ws_t ws, const double* D, const double* T, int n, int b, int 
 #define BTA_OPT_TILE_UPDATE 1
 #define BTA_OPT_TILE_GROUPED 2
 /* Panel factorization of bta_potrf: 0 = automatic (2 for b > 64, else the
- * whole factorization as one workgroup), 1 = one launch per 64-wide tile column, 2 = one persistent dataflow launch per block (a chain
+ * whole factorization as one workgroup where a <= 32), 1 = one launch per
+ * 64-wide tile column, 2 = one persistent dataflow launch per block (a chain
  * workgroup on the diagonal plus helper workgroups running a dependency-
  * levelled task list).  BTA_OPT_FLOW_HELPERS sets the helper count (0 =
  * automatic: half the device's resident capacity, less one) and

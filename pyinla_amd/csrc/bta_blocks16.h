@@ -17,6 +17,17 @@ __device__ __forceinline__ f64x4 gload16(const double* g, int ld, int r0, int c0
   }
   return v;
 }
+// The first 16x16 block, its upper triangle from the lower one.
+__device__ __forceinline__ f64x4 gload16_sym(const double* g, int ld, int rows) {
+  const int lane = threadIdx.x & 63, j = lane & 15;
+  f64x4 v;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int i = 4 * q + (lane >> 4), r = max(i, j), c = min(i, j);
+    v[q] = r < rows ? gview(g)[(int64_t)r * ld + c] : 0.0;
+  }
+  return v;
+}
 __device__ __forceinline__ void gstore16(double* g, int ld, int r0, int c0, int rows, int cols, f64x4 v) {
   const int lane = threadIdx.x & 63, c = c0 + (lane & 15);
 #pragma unroll
@@ -32,13 +43,15 @@ struct Blocks {
   f64x4 v[U];
   int row[U], col[U], n;
   // the wave's share of a lower triangle of m block rows, or of m x c blocks,
-  // dealt one by one starting with wave `first`
-  __device__ __forceinline__ void deal(int m, int c, bool lower, int first) {
-    const int me = (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) - first) & (W - 1), total = lower ? m * (m + 1) / 2 : m * c;
+  // dealt one by one over the last `waves` waves, starting `first` after the
+  // first of them, block number `skip` the first to go
+  __device__ __forceinline__ void deal(int m, int c, bool lower, int first, int waves = W, int skip = 0) {
+    const int me = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) - (W - waves);
+    const int at = me - first < 0 ? me - first + waves : me - first, total = lower ? m * (m + 1) / 2 : m * c;
     n = 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int e = me + W * u;
+      const int e = skip + at + waves * u;
       int r = 0, k = e;
       while (k >= (lower ? r + 1 : max(c, 1))) {
         k -= lower ? r + 1 : c;
@@ -46,7 +59,7 @@ struct Blocks {
       }
       row[u] = 16 * r;
       col[u] = 16 * k;
-      n += e < total;
+      n += me >= 0 && e < total;
     }
   }
   __device__ __forceinline__ void load(const double* g, int ld, int rows, int cols) {

@@ -254,9 +254,10 @@ __global__ void k_begin_batch(const ProbDesc* probs, int nprob) {
 // and on passing the tile through memory than on the arithmetic.  Everything a
 // block hands to the next one stays in LDS or registers; the next block's
 // operands are loaded while this one is factored, and only the 16-wide block
-// columns that b has are factored.  Bound by the chain of pivots.  Measured on
-// MI355X, us per block (a = 6), against the two launches: b = 16 8.0 / 24.8, b = 40
-// 15.3 / 26.6, b = 64 18.2 / 26.3.
+// columns that b has are factored.  Arrows above 32 rows would need more
+// registers and gained nothing (a = 64: 25.2 against 26.4 us).  Bound by the chain of pivots.  Measured on
+// MI355X, us per block (a = 6), against the two launches: b = 16 7.1 / 24.8, b = 40
+// 14.4 / 26.6, b = 64 17.9 / 26.3.
 struct ChainArgs {
   double *D, *L, *B, *T;
   double* Winv;     // n inverse tiles
@@ -275,23 +276,43 @@ __global__ void __launch_bounds__(BTA_THREADS, 1) k_chain64(ChainArgs p) {
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   // The 16x16 blocks of each product, dealt over the waves so that the four
   // come out even: L_i = X W^T takes a block row per wave (10 of 16 products),
-  // D_{i+1} its lower triangle (3, 3, 2, 2), then the arrow's.
-  Blocks<4> xb, yb, bn;
-  Blocks<3> d, t;
+  // D_{i+1}'s first block wave 0, which factors it while the
+  // others update the rest of the lower triangle and the arrow's blocks.
+  Blocks<4> xb;
+  Blocks<2> yb;
+  Blocks<3> d, bn;
+  Blocks<1> t;
   xb.n = wv < nb ? nb : 0;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     xb.row[u] = 16 * wv;
     xb.col[u] = 16 * u;
   }
-  d.deal(nb, nb, true, 0);
+  d.deal(nb, nb, true, 0, 3, 1);
   yb.deal(na, nb, false, 3);
-  bn.deal(na, nb, false, 2);
-  t.deal(na, na, true, 2);
+  bn.deal(na, nb, false, 1, 3);
+  t.deal(na, na, true, 2, 3);
   lds_load_tile(s, p.D, b, b, b);
   if (a > 0) {
     lds_load_tile(y, p.B, b, a, b);
     t.load(p.T, a, a, a);
+  }
+  __syncthreads();
+  if (b == 64) clear_upper_blocks(s, w, threadIdx.x, BTA_THREADS);  // later blocks leave them so
+  // wave 0: the first 16x16 block of the next D, the identity past b, and then
+  // its factor and inverse
+  f64x4 d0, e0;
+  auto factor_first = [&] {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = 4 * q + (lane >> 4), c = lane & 15;
+      if (r >= b || c >= b) d0[q] = r == c ? 1.0 : 0.0;
+    }
+    chol16_inv16(d0, e0);
+  };
+  if (wv == 0) {
+    d0 = gload16_sym(p.D, b, b);
+    factor_first();
   }
   __syncthreads();
   for (int i = 0; i < n; ++i) {
@@ -299,17 +320,20 @@ __global__ void __launch_bounds__(BTA_THREADS, 1) k_chain64(ChainArgs p) {
     double* Di = p.D + i * bb;
     double* Li = p.L + i * bb;
     double* Bi = p.B + i * ab;
-    TilePrefetch pl;
-    if (next) {
-      pl.load(Li, b, 0, b, b);
-      d.load(Di + bb, b, b, b);
-      if (a > 0) bn.load(Bi + ab, b, a, b);
-    }
     if (b < 64) {
       tile_chol_pad(s, w, b);
       lds_barrier();
     }
-    tile_chol_blocks<false>(s, w, b, [] {}, nb);
+    if (wv == 0) store_chol16(d0, e0, s, w, 0);
+    lds_barrier();
+    TilePrefetch pl;
+    if (next) {
+      pl.load(Li, b, 0, b, b);
+      if (wv == 0) d0 = gload16_sym(Di + bb, b, b);
+      d.load(Di + bb, b, b, b);
+      if (a > 0) bn.load(Bi + ab, b, a, b);
+    }
+    tile_chol_blocks<true>(s, w, b, [] {}, nb);
     const double lii = s[lane * BTA_LDS_LD + lane];
     if (next) pl.store(x, 0);
     for (int r = wv; r < 64; r += 4) {
@@ -335,14 +359,21 @@ __global__ void __launch_bounds__(BTA_THREADS, 1) k_chain64(ChainArgs p) {
       yb.store(Bi, b, a, b);
     }
     lds_barrier();
-#pragma unroll
-    for (int k = 0; k < 64; k += 16) {
-      if (k >= b) break;
+    if (wv == 0) {
       if (next) {
-        d.product<true, 0, 0>(x, x, k);
-        bn.product<true, 0, 0>(y, x, k);
+        for (int k = 0; k < b; k += 16) d0 = mma16x16<true, 0>(x, 0, k, x, 0, k, d0);
+        factor_first();
       }
-      t.product<true, 0, 0>(y, y, k);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 64; k += 16) {
+        if (k >= b) break;
+        if (next) {
+          d.product<true, 0, 0>(x, x, k);
+          bn.product<true, 0, 0>(y, x, k);
+        }
+        t.product<true, 0, 0>(y, y, k);
+      }
     }
     if (wv == 3) {
       const TileCholResult res = tile_log_pivots(lii, b);
@@ -359,7 +390,7 @@ __global__ void __launch_bounds__(BTA_THREADS, 1) k_chain64(ChainArgs p) {
     lds_barrier();
   }
 #pragma unroll
-  for (int u = 0; u < 3; ++u)
+  for (int u = 0; u < 1; ++u)
     if (u < t.n)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -665,7 +696,7 @@ int potrf_enqueue(Workspace& ws, double* D, double* L, double* B, double* T, int
   const bool flow = use_flow(ws, b) && ws.flow && ws.flow->nT == nT && ws.flow_sched && ws.flow_sched->nTa == nTa;
   if (use_flow(ws, b) && !flow) return (int)hipErrorNotReady;  // potrf_prepare not run for this shape
   hipLaunchKernelGGL(k_begin_call, dim3(1), dim3(64), 0, st, ws.epoch, ws.info, ws.err);
-  const bool chain = b <= 64 && a <= 64 && ws.panel_mode == 0 && !use_plan;
+  const bool chain = b <= 64 && a <= 32 && ws.panel_mode == 0 && !use_plan;
   if (chain) {
     TimedScope ts(ws, KC_PANEL, st);
     hipLaunchKernelGGL(k_chain64, dim3(1), dim3(BTA_THREADS), 0, st,
