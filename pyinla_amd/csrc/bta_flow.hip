@@ -776,10 +776,11 @@ __device__ __forceinline__ void flow_chain(const FlowArgs& p, unsigned long long
     if (k + 2 < nT && threadIdx.x < 2) hv = flag_value(hflag(p, k + 1, threadIdx.x), tag);
     if (threadIdx.x < 64) {
       const bool all = __ballot(hv != tag) == 0;
-      if (threadIdx.x == 0) ok_sh[0] = all ? 1 : 0;
+      if (threadIdx.x == 0) ok_sh[2] = all ? 1 : 0;
     }
     flow_publish(wflag(p, k + 1), tag);
-    ready = ok_sh[0] != 0;
+    // a word of its own: flow_wait2 writes ok_sh[0] with no barrier after this read
+    ready = ok_sh[2] != 0;
   }
   chain_store_l(p, nT - 1, sA);
   if (w == 0) chain_log(p, nT - 1, sA[lane * BTA_LDS_LD + lane]);
@@ -1067,7 +1068,7 @@ __device__ __forceinline__ void flow_helper(const FlowArgs& p, int h, unsigned l
 __global__ void __launch_bounds__(BTA_THREADS, 2) k_panel_flow(FlowArgs p) {
   __shared__ double sA[64 * BTA_LDS_LD];
   __shared__ double sB[64 * BTA_LDS_LD];
-  __shared__ int ok_sh[2];
+  __shared__ int ok_sh[3];
   const unsigned long long tag = (p.epoch[0] << 20) | (unsigned long long)p.blk;
   if (blockIdx.x == 0) flow_chain(p, tag, sA, sB, ok_sh);
   else flow_helper(p, blockIdx.x - 1, tag, sA, sB);
@@ -1210,7 +1211,7 @@ void flow_launch_block(const Workspace& ws, const FlowPlan& fp, const FlowSched&
 __global__ void __launch_bounds__(BTA_THREADS, 2) k_panel_flow_batched(FlowBatch fb) {
   __shared__ double sA[64 * BTA_LDS_LD];
   __shared__ double sB[64 * BTA_LDS_LD];
-  __shared__ int ok_sh[2];
+  __shared__ int ok_sh[3];
   const int wg = (int)blockIdx.x;
   int pos = wg;  // position in the entries' ranges of `begin`
   if (fb.iso) {
