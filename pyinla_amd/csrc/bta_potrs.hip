@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "bta_internal.h"
+#include "bta_sweep_walk.h"
 
 namespace bta {
 
@@ -126,20 +127,8 @@ __device__ __forceinline__ double sum8(double v) {
 
 // -------------------------------------------------------- several workgroups
 //
-// A sweep is a list of products ("stages"): per block the coupling with the
-// block before it (L_{i-1} y_{i-1}, or L_i^T x_{i+1} + B_i^T x_a) and the
-// product with W_i.  A stage is cut into work items; seat k of the launch owns
-// items k, k + seats, ... of every stage.  (Items taken by ticket instead: two
-// items of one stage often went to the same workgroup, which then ended 6 us
-// after the others at b = 1600.)
-//
-// The launch must end whatever number of its workgroups the device keeps
-// resident beside other kernels.  A workgroup therefore claims its seat when it
-// starts, and one that has waited for stage 0 for 10 ms (another sweep of the
-// same size would have made room by then) claims the seats whose items are
-// still missing there: it runs their items too, in every stage, and the
-// workgroups they were meant for find them taken and end.  Once stage 0 is
-// complete every seat belongs to a running workgroup.
+// The items of a sweep, who runs them and why the launch always ends:
+// bta_sweep_walk.h.
 //
 // Hand-over: every stage has a vector of its own, filled with kPending before
 // the launch; an item stores its outputs there with write-through stores (whole
@@ -153,8 +142,8 @@ __device__ __forceinline__ double sum8(double v) {
 // and by k_sweep_finish; strips of 8 columns fetched every line twice (1.8
 // times the bytes).  A wave has up to U loads of its item in flight before the
 // vector arrives; larger blocks run in rounds.
+
 // What the two kinds of waves of a workgroup share.
-constexpr int kSeats = 512;  // at most
 template <int R, int U, bool T>
 struct SweepLds {
   static constexpr int RK = (T ? 64 : 128) * U;   // vector elements per round
@@ -164,119 +153,78 @@ struct SweepLds {
   double red[T ? 8 * NO * R : NO * R];
   double xa[T ? 64 * R : 1];
   int seat[kSeats];  // the seats of this workgroup
-  int victim[2];     // a seat found missing by a wait for stage 0 (kSeats: none)
-  int got;           // what became of it: 0 wait again, 1 taken over, 2 the launch is failing
+  int victim;        // at the gate: distance from the own seat to a free one (kSeats: none)
+  int got;           // the seat that was taken over (-1: another workgroup has it)
   int dead;          // the own seat was taken
 };
 
-// Geometry of an item.
-template <bool T>
-struct SweepItem {
-  int stage, part, i, out0, hf;
-  bool isw, hasm;
-  int kbeg, kend, kall;  // vector range (forward: kend is that of the item's last row)
-  __device__ __forceinline__ SweepItem(const SweepArgs& p, int stage_, int part_) : stage(stage_), part(part_) {
-    constexpr int NO = T ? 16 : 8;
-    // forward: W(0), L(0), W(1), ...; backward: the last block's arrow term
-    // when there is an arrow, W(n-1), L(n-2), W(n-2), ...
-    const int first = (T && p.a > 0) ? 0 : 1;
-    isw = ((stage + first) & 1) != 0;  // product with W
-    const int step = (stage + first) >> 1;
-    i = T ? p.n - 1 - step : step;
-    hasm = isw || !T || i < p.n - 1;  // the arrow term alone has no matrix
-    hf = T ? part & 1 : 0;            // half of the rows
-    out0 = NO * (T ? part >> 1 : part);
-    kbeg = 0;
-    kend = !hasm ? 0 : ((!T && isw) ? min(out0 + NO, p.b) : p.b);
-    if (T && hasm) {  // W is zero above its diagonal
-      const int lo = isw ? out0 : 0, mid = (lo + p.b + 1) >> 1;
-      kbeg = hf ? mid : lo;
-      kend = hf ? p.b : mid;
+constexpr unsigned kPatience = 1000000;  // s_memrealtime ticks (100 MHz): 10 ms
+
+// The claims of the seats that a waiting thread looks after.
+template <int NP>
+struct SweepClaims {
+  static constexpr int N = kSeats / (64 * NP);
+  unsigned c[N];
+  __device__ __forceinline__ void load(const SweepArgs& p, int t) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      c[j] = __hip_atomic_load(p.claims + min(t + 64 * NP * j, p.seats - 1), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  // Distance from the own seat to a free one, kSeats if all are claimed: each
+  // workgroup takes over another one first.
+  __device__ __forceinline__ int free_seat(const SweepArgs& p, int t, int own) const {
+    int d = kSeats;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int s = min(t + 64 * NP * j, p.seats - 1), e = s - own;
+      if (c[j] == 0) d = min(d, e < 0 ? e + p.seats : e);
     }
-    kall = kend;
+    return d;
   }
 };
 
-// The items of a workgroup in order, the same in all its threads: its seats'
-// items of a stage, then those of the next stage.  A seat taken over while the
-// first item of stage 1 waits has its stage-0 items run before that item.
-struct SweepWalk {
-  int stages, parts, seats, count = 1, stage = 0, q = 0, part, resume = -1;
-  __device__ __forceinline__ SweepWalk(const SweepArgs& p, int stages_, int seat)
-      : stages(stages_), parts(p.parts), seats(p.seats), part(seat) {}
-  bool fresh = false;  // the walk already stands at the item to run
-  template <class Lds>
-  __device__ __forceinline__ bool more(const Lds& l) {
-    if (fresh) {
-      fresh = false;
-      return true;
-    }
-    part += seats;
-    if (part < parts) return true;
-    if (resume >= 0) {  // the late seat's stage-0 items are done
-      stage = 1;
-      q = 0;
-      part = resume;
-      resume = -1;
-      return true;
-    }
-    if (++q == count) {
-      q = 0;
-      ++stage;
-    }
-    part = __builtin_amdgcn_readfirstlane(l.seat[q]);
-    return stage < stages;
-  }
-  __device__ __forceinline__ void take_over(int seat) {
-    resume = part;
-    stage = 0;
-    q = count++;
-    part = seat;
-    fresh = true;
-  }
-};
-
-// End of a wait, called by all threads.  Stage 1 waits for stage 0 and may find
-// seats missing (`seat`, kSeats if none): returns 0 = everything arrived, 1 =
-// wait again, 2 = the walk goes on with the late seat.  Later waits only end.
-// `turn` alternates between two words, so that one is still readable while the
-// next wait runs.
-template <class Lds, class Claim>
-__device__ __forceinline__ int sweep_settle(Lds& l, SweepWalk& walk, int& turn, int seat, bool chief, Claim&& claim) {
-  if (walk.stage != 1) {
+// The gate, called by all threads: returns once every seat is claimed, or with
+// the walk at the stage-0 items of a seat this workgroup has taken over.  `look`:
+// what this thread finds (kSeats: no free seat), after some time of waiting.
+template <class Lds, class Look>
+__device__ __forceinline__ void sweep_gate(const SweepArgs& p, Lds& l, SweepWalk& walk, int own, bool chief,
+                                           Look&& look) {
+  for (bool first = walk.count == 1;; first = false) {
+    const int d = look(first);
+    if (d < kSeats) atomicMin(&l.victim, d);
     lds_barrier();
-    return 0;
+    const int v = __builtin_amdgcn_readfirstlane(l.victim);
+    if (v >= kSeats) {
+      walk.open = true;
+      return;
+    }
+    lds_barrier();
+    if (chief) {
+      const int s = own + v < p.seats ? own + v : own + v - p.seats;
+      l.victim = kSeats;
+      l.got = claim_seat(p.claims + s) == 0 ? s : -1;
+      if (l.got >= 0) l.seat[walk.count] = s;
+    }
+    lds_barrier();
+    const int s = __builtin_amdgcn_readfirstlane(l.got);
+    if (s >= 0) {
+      walk.take_over(s);
+      return;
+    }
   }
-  turn ^= 1;
-  if (seat < kSeats) atomicMin(&l.victim[turn], seat);
-  lds_barrier();
-  const int v = __builtin_amdgcn_readfirstlane(l.victim[turn]);
-  if (v >= kSeats) return 0;
-  lds_barrier();
-  if (chief) {
-    l.got = claim(v);
-    l.victim[turn] = kSeats;
-    if (l.got == 1) l.seat[walk.count] = v;
-  }
-  lds_barrier();
-  const int got = __builtin_amdgcn_readfirstlane(l.got);
-  lds_barrier();
-  if (got == 1) walk.take_over(v);
-  return got == 0 ? 1 : (got == 1 ? 2 : 0);
 }
 
 // Brings elements [ks, ks + cnt / R) of the vector before stage g.stage into
-// LDS, by threads t of nt; `waiting` says whether to go on waiting.  Returns
-// the seat of an element that did not arrive (kSeats: all did).
+// LDS, by threads t of nt; `waiting` says whether to go on waiting.
 template <int R, int U, bool T, class Wait>
-__device__ __forceinline__ int sweep_stage(const SweepArgs& p, SweepLds<R, U, T>& l, const SweepItem<T>& g, int ks,
-                                           int cnt, int t, int nt, Wait&& waiting) {
+__device__ __forceinline__ void sweep_stage(const SweepArgs& p, SweepLds<R, U, T>& l, const SweepItem<T>& g, int ks,
+                                            int cnt, int t, int nt, Wait&& waiting) {
   using Lds = SweepLds<R, U, T>;
   const int64_t half = vec_len(p.b, R);
   const double* sr = p.vec + g.stage * (T ? 2 * half : half) + (int64_t)ks * R;  // stage s writes vector s + 1
   // loads in flight per thread and vector: one batch brings a round's vector
   constexpr int Q = R > 1 ? (T ? 4 : 8) : U / 2;
-  int missing = kSeats;
   for (int e0 = t; e0 < cnt; e0 += Q * nt) {
     unsigned long long v[Q], h[T ? Q : 1];
     auto pending = [&]() {
@@ -297,34 +245,23 @@ __device__ __forceinline__ int sweep_stage(const SweepArgs& p, SweepLds<R, U, T>
     for (int q = 0; q < Q; ++q)
       if (const int e = e0 + q * nt; e < cnt) {
         double x = __longlong_as_double((long long)v[q]);
-        const int o = (ks + e / R) / Lds::NO;  // the item that writes element e
-        if (v[q] == kPending) missing = (T ? 2 * o : o) % p.seats;
-        if constexpr (T) {
-          x += __longlong_as_double((long long)h[q]);
-          if (h[q] == kPending) missing = (2 * o + 1) % p.seats;
-        }
+        if constexpr (T) x += __longlong_as_double((long long)h[q]);
         l.v[e % R * Lds::LV + e / R] = x;
       }
   }
-  return missing;
 }
 
-constexpr unsigned kPatience = 1000000;  // s_memrealtime ticks (100 MHz): 10 ms
-
-// Bound on a wait of a thread.  In stage 1 it ends after `patience`
-// s_memrealtime ticks (100 MHz) to look for late seats; for good, with err,
-// after spin_ticks, or once another workgroup has raised err.
+// Bound on a wait of a thread: it ends, with err, after spin_ticks, or once
+// another workgroup has raised err (looked at after 10 ms: polled by everyone from
+// the start, that one word would be a hot spot).
 struct SweepWait {
   const SweepArgs& p;
-  int stage;
-  unsigned patience;
   unsigned long long t0 = 0;
   __device__ __forceinline__ bool operator()() {
     __builtin_amdgcn_s_sleep(1);
     const unsigned long long now = __builtin_amdgcn_s_memrealtime();
     if (t0 == 0) t0 = now;
-    if (now - t0 < patience) return true;
-    if (stage == 1) return false;
+    if (now - t0 < kPatience) return true;
     if (__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0) return false;
     if (now - t0 < p.spin_ticks) return true;
     __hip_atomic_fetch_or(p.err, 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -340,38 +277,32 @@ template <int R, int U, bool T, int NP>
 __device__ __forceinline__ void sweep_poller(const SweepArgs& p, SweepLds<R, U, T>& l, int stages, int own) {
   using Lds = SweepLds<R, U, T>;
   const int t = (int)threadIdx.x - kSweepThreads;
-  SweepWalk walk(p, stages, own);
-  unsigned patience = kPatience;
-  unsigned long long t1 = 0;
-  int turn = 0;
-  do {
-    const SweepItem<T> g(p, walk.stage, walk.part);
-    auto claim = [&](int v) -> int {  // by thread 0
-      const unsigned long long now = __builtin_amdgcn_s_memrealtime();
-      if (t1 == 0) t1 = now;
-      if (now - t1 > p.spin_ticks) __hip_atomic_fetch_or(p.err, 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      if (__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0) return 2;
-      return claim_seat(p.claims + v) == 0 ? 1 : 0;
-    };
-    auto settle = [&](int seat) -> int {
-      const int r = sweep_settle(l, walk, turn, seat, t == 0, claim);
-      if (r == 2) patience = kPatience / 100;  // do not wait as long for the next one
-      return r;
-    };
-    int r = 0;
-    for (int ks = g.kbeg; ks < g.kall && r == 0; ks += Lds::RK) {
-      if (ks > g.kbeg) lds_barrier();  // the previous round's reads are done
-      do {
-        const int missing = sweep_stage<R, U, T>(p, l, g, ks, min(Lds::RK, g.kall - ks) * R, R > 1 ? threadIdx.x : t,
-                                                 R > 1 ? kSweepThreads + 64 * NP : 64 * NP,
-                                                 SweepWait{p, g.stage, patience});
-        r = settle(missing);
-      } while (r == 1);
+  SweepWalk walk(stages, p.parts, p.seats, own);
+  // the claims, loaded in stage 0 beside the products and looked at from the gate on
+  SweepClaims<NP> claims;
+  auto look = [&](bool first) {
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    int d;
+    while ((d = claims.free_seat(p, t, own)) < kSeats &&
+           __builtin_amdgcn_s_memrealtime() - t0 < (first ? kPatience : kPatience / 100)) {
+      __builtin_amdgcn_s_sleep(1);
+      claims.load(p, t);
     }
-    if (r == 2) continue;
+    return d;
+  };
+  do {
+    if (walk.at_gate()) sweep_gate(p, l, walk, own, t == 0, look);
+    const SweepItem<T> g(p.n, p.b, p.a, walk.stage, walk.part);
+    for (int ks = g.kbeg; ks < g.kend; ks += Lds::RK) {
+      if (ks > g.kbeg) lds_barrier();  // the previous round's reads are done
+      sweep_stage<R, U, T>(p, l, g, ks, min(Lds::RK, g.kend - ks) * R, R > 1 ? threadIdx.x : t,
+                           R > 1 ? kSweepThreads + 64 * NP : 64 * NP, SweepWait{p});
+      lds_barrier();
+    }
+    if (walk.stage == 0) claims.load(p, t);
     lds_barrier();  // [red]
     lds_barrier();  // [end]
-  } while (walk.more(l));
+  } while (walk.more(l.seat));
 }
 
 // Waves that multiply: 8 of them, each with up to U 16-byte loads of the
@@ -383,11 +314,10 @@ __device__ __forceinline__ void sweep_worker(const SweepArgs& p, SweepLds<R, U, 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = p.b, a = p.a;
   const int64_t half = vec_len(b, R), vlen = T ? 2 * half : half;
-  SweepWalk walk(p, stages, own);
-  int turn = 0;
-  auto settle = [&](int seat) { return sweep_settle(l, walk, turn, seat, false, [](int) { return 0; }); };
+  SweepWalk walk(stages, p.parts, p.seats, own);
   do {
-    const SweepItem<T> g(p, walk.stage, walk.part);
+    if (walk.at_gate()) sweep_gate(p, l, walk, own, false, [](bool) { return kSeats; });
+    const SweepItem<T> g(p.n, b, a, walk.stage, walk.part);
     const int i = g.i;
     const double* M = g.isw || !g.hasm ? p.W + (int64_t)i * b * b : p.L + (int64_t)(T ? i : i - 1) * b * b;
     const int row = T ? g.out0 : g.out0 + w;  // this wave's output row / the strip's first column
@@ -420,20 +350,14 @@ __device__ __forceinline__ void sweep_worker(const SweepArgs& p, SweepLds<R, U, 
     double acc[NA];
 #pragma unroll
     for (int q = 0; q < NA; ++q) acc[q] = 0.0;
-    int r = 0;
-    for (int ks = g.kbeg; ks < g.kall && r == 0; ks += RK) {
+    for (int ks = g.kbeg; ks < g.kend; ks += RK) {
       if (ks > g.kbeg) {
         lds_barrier();
         fetch(ks);
       }
-      do {
-        int missing = kSeats;
-        if constexpr (R > 1)
-          missing = sweep_stage<R, U, T>(p, l, g, ks, min(RK, g.kall - ks) * R, tid, kSweepThreads + 64 * NP,
-                                         SweepWait{p, g.stage, kPatience});
-        r = settle(missing);
-      } while (r == 1);
-      if (r == 2) break;
+      if constexpr (R > 1)
+        sweep_stage<R, U, T>(p, l, g, ks, min(RK, g.kend - ks) * R, tid, kSweepThreads + 64 * NP, SweepWait{p});
+      lds_barrier();
       const int ke = min(ks + RK, kend);
       // tests only every few steps: the LDS reads of a step overlap the products
       // of the one before
@@ -467,7 +391,6 @@ __device__ __forceinline__ void sweep_worker(const SweepArgs& p, SweepLds<R, U, 
         }
       }
     }
-    if (r == 2) continue;
     double out = 0.0;
     if constexpr (T) {
       if (arrow) {
@@ -507,19 +430,19 @@ __device__ __forceinline__ void sweep_worker(const SweepArgs& p, SweepLds<R, U, 
       if (!T && g.isw && orc < p.nr) p.X[((int64_t)i * b + orow) * p.ldx + orc] = v;
     }
     lds_barrier();  // [end]: v and red are free for the next item
-  } while (walk.more(l));
+  } while (walk.more(l.seat));
 }
 
 template <int R, int U, bool T, int NP>
 __global__ void __launch_bounds__(kSweepThreads + 64 * NP, 4) k_sweep(SweepArgs p) {
   __shared__ SweepLds<R, U, T> l;
-  const int stages = 2 * p.n - ((T && p.a > 0) ? 0 : 1);
+  const int stages = sweep_stages(p.n, p.a, T);
   const int group = (int)blockIdx.x / p.seats, own = (int)blockIdx.x - group * p.seats;
   p.enter_group(R, group);
   if (threadIdx.x == 0) {
     l.dead = claim_seat(p.claims + own) != 0;
     l.seat[0] = own;
-    l.victim[0] = l.victim[1] = kSeats;
+    l.victim = kSeats;
   }
   if constexpr (T)
     for (int e = threadIdx.x; e < p.a * R; e += blockDim.x)
@@ -795,13 +718,13 @@ __global__ void __launch_bounds__(BTA_THREADS) k_sweep_arrow(SweepArgs p, const 
 template <int R, int U, int NP>
 int sweep_group(Workspace& ws, SweepArgs p, const double* x0, double* Xtip, int tip, int trans, int groups,
                 hipStream_t st) {
-  p.parts = trans ? 2 * ((p.b + 15) / 16) : (p.b + 7) / 8;
+  p.parts = sweep_parts(p.b, trans);
   // one workgroup per CU; two where a product has more items than that (their
   // rounds of loads then overlap: b = 4500 27 / 37 us per product forward /
   // backward against 35 / 48), which only the small R = 1, U = 8 form has the
   // registers for
   p.seats = std::min(p.parts, std::min(R == 1 && U == 8 && p.b > 2048 ? 2 * ws.cus : ws.cus, kSeats));
-  const int64_t products = 2 * (int64_t)p.n - ((trans && p.a > 0) ? 0 : 1), len = vec_len(p.b, R);
+  const int64_t products = sweep_stages(p.n, p.a, trans), len = vec_len(p.b, R);
   const int64_t vectors = (products + 1) * (trans ? 2 : 1);
   p.gstride = vectors * len + kSeats / 2;
   groups = std::max(1, std::min({groups, (p.nr + R - 1) / R, ws.cus / p.seats}));
