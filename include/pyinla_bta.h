@@ -137,7 +137,8 @@ int bta_batch_destroy(bta_batch_t batch);
  *   logdet : 2 * sum log diag of the factor (the reference's
  *            SerinvSolver.logdet, structured_solver.py:151-166; for a == 0 the
  *            tip is excluded, as sparsity="bt" does);
- *   err    : BTA_E_TIMEOUT if a bounded wait expired, else 0.
+ *   err    : BTA_E_TIMEOUT if a bounded wait of it, or of a sweep that neither
+ *            this call nor bta_solve_status has reported yet, expired, else 0.
  * Any output pointer may be NULL. */
 int bta_ws_status(bta_ws_t ws, int64_t* info, double* logdet, int* err, void* stream);
 
@@ -198,6 +199,8 @@ int bta_logdet(bta_ws_t ws, const double* D, const double* T, int n, int b, int 
  * panel and the update follows as one grouped-GEMM launch; 0 (default) =
  * automatic (1 up to 48 tile columns, b <= 3072, else 2). */
 #define BTA_OPT_FLOW_FOLD 10
+/* Bound on one in-kernel wait of a triangular sweep in ms (default 20000). */
+#define BTA_OPT_SOLVE_WAIT 11
 int bta_ws_set_option(bta_ws_t ws, int option, int value);
 
 /* Host-only diagnostic (no reference counterpart): the helper task lists of
@@ -229,9 +232,16 @@ int bta_ws_get_timing(bta_ws_t ws, int kclass, double* total_ms, int64_t* count)
  * (ldrhs >= nrhs, any nrhs).  The first call after a factorization
  * also forms W_i = D_i^-1 for every block in the reserved buffer
  * (BTA_WS_SOLVE or BTA_WS_SELINV; BTA_E_NORES without it).  Launched
- * directly, never from a recorded graph. */
+ * directly, never from a recorded graph.  For b > 64 the workgroups of a sweep
+ * wait for each other, each wait bounded (BTA_OPT_SOLVE_WAIT): a sweep that gave
+ * up leaves NaN in rhs and is reported by bta_solve_status; the factor stays
+ * usable. */
 int bta_potrs(bta_ws_t ws, double* D, double* L, double* B, double* T, int n, int b, int a,
               double* rhs, int nrhs, int ldrhs, int trans, void* stream);
+/* Synchronise the stream; err = BTA_E_TIMEOUT if a sweep of the workspace gave up
+ * since this (or bta_ws_status) was last called, else 0.  Costs no copy: the
+ * sweeps raise a word in host memory.  No reference counterpart. */
+int bta_solve_status(bta_ws_t ws, int* err, void* stream);
 
 /* In-place selected inversion: the factor blocks are overwritten by the
  * blocks of Sigma = Q^-1 on the BTA pattern -- D[i] <- Sigma_ii (full

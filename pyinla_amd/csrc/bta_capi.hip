@@ -246,13 +246,15 @@ int bta_ws_create(int device, int n, int b, int a, int flags, bta_ws_t* out) {
   w.epoch = u + nflags;
   w.info = u + nflags + 1;
   w.err = reinterpret_cast<int*>(u + nflags + 2);
+  w.sweep_fail = reinterpret_cast<int*>(u + nflags + 4);
   w.sweep_count = reinterpret_cast<int*>(u + nflags + 6);
   w.wait_ticks = bta::flow_spin_ticks(device, 20.0);
   if (hipDeviceGetAttribute(&w.cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || w.cus < 1)
     w.cus = 1;
   w.base_bytes = nd * sizeof(double) + (nflags + 2) * sizeof(unsigned long long) + 64;
-  int rc = 0;
-  if (bta::flow_wanted(w, b)) rc = bta::flow_alloc(w);
+  int rc = (int)hipHostMalloc(reinterpret_cast<void**>(&w.solve_err), sizeof(int), hipHostMallocDefault);
+  if (!rc) *w.solve_err = 0;
+  if (!rc && bta::flow_wanted(w, b)) rc = bta::flow_alloc(w);
   if (!rc && (flags & (BTA_WS_SOLVE | BTA_WS_SELINV))) rc = bta_ws_reserve(ws, flags & (BTA_WS_SOLVE | BTA_WS_SELINV));
   if (rc) {
     bta_ws_destroy(ws);
@@ -284,6 +286,7 @@ int bta_ws_destroy(bta_ws_t ws) {
   if (ws->w.gfull) hipFree(ws->w.gfull);
   if (ws->w.flags) hipFree(ws->w.flags);
   if (ws->w.wfull) hipFree(ws->w.wfull);
+  if (ws->w.solve_err) hipHostFree(ws->w.solve_err);
   delete ws;
   return 0;
 }
@@ -481,6 +484,11 @@ int bta_batch_destroy(bta_batch_t bt) {
   return 0;
 }
 
+// Whether a wait of a sweep has given up since this was last asked.
+static bool take_solve_error(bta::Workspace& w) {
+  return __atomic_exchange_n(w.solve_err, 0, __ATOMIC_RELAXED) != 0;
+}
+
 int bta_ws_status(bta_ws_t ws, int64_t* info, double* logdet, int* err, void* stream) {
   if (!ws) return BTA_E_ARG;
   hipStream_t st = as_stream(stream);
@@ -494,7 +502,16 @@ int bta_ws_status(bta_ws_t ws, int64_t* info, double* logdet, int* err, void* st
   if ((e = hipMemcpy(&ld, ws->w.logdet, sizeof(ld), hipMemcpyDeviceToHost)) != hipSuccess) return (int)e;
   if (info) *info = (inf == bta::kInfoNone) ? 0 : (int64_t)inf + 1;
   if (logdet) *logdet = ld;
-  if (err) *err = er ? BTA_E_TIMEOUT : 0;
+  const bool solve_failed = take_solve_error(ws->w);
+  if (err) *err = er || solve_failed ? BTA_E_TIMEOUT : 0;
+  return 0;
+}
+
+int bta_solve_status(bta_ws_t ws, int* err, void* stream) {
+  if (!ws || !err) return BTA_E_ARG;
+  const hipError_t e = hipStreamSynchronize(as_stream(stream));
+  if (e != hipSuccess) return (int)e;
+  *err = take_solve_error(ws->w) ? BTA_E_TIMEOUT : 0;
   return 0;
 }
 
@@ -529,6 +546,7 @@ int bta_ws_set_option(bta_ws_t ws, int option, int value) {
   if (option == BTA_OPT_FLOW_NEAR && (value < 1 || value > 64)) return BTA_E_ARG;
   if (option == BTA_OPT_GEMM_KERNEL && value != 0 && value != 1) return BTA_E_ARG;
   if (option == BTA_OPT_FLOW_FOLD && (value < 0 || value > 2)) return BTA_E_ARG;
+  if (option == BTA_OPT_SOLVE_WAIT && value < 0) return BTA_E_ARG;
   std::lock_guard<std::mutex> g(ws->mu);
   if (option == BTA_OPT_TILE_UPDATE) ws->w.tile_update = value;
   else if (option == BTA_OPT_TILE_GROUPED) ws->w.tile_grouped = value;
@@ -546,6 +564,7 @@ int bta_ws_set_option(bta_ws_t ws, int option, int value) {
   else if (option == BTA_OPT_FLOW_NEAR) ws->w.flow_near = value;
   else if (option == BTA_OPT_GEMM_KERNEL) ws->w.gemm_variant = value;
   else if (option == BTA_OPT_FLOW_FOLD) ws->w.flow_fold = value;
+  else if (option == BTA_OPT_SOLVE_WAIT) ws->w.wait_ticks = bta::flow_spin_ticks(ws->w.device, 1e-3 * value);
   else return BTA_E_ARG;
   // recorded graphs embed the old launch shapes
   drop_graphs(ws);

@@ -135,6 +135,8 @@ struct Workspace {
   double* tinv = nullptr;               // 64 x 64: inverse of the tip factor
   unsigned long long spin_limit = 1ull << 24;
   int* sweep_count = nullptr;           // arrow partial sums counted (zero between launches)
+  int* sweep_fail = nullptr;            // a wait of the running sweep gave up
+  int* solve_err = nullptr;             // pinned host word: a wait of a sweep gave up since it was last read
   unsigned long long wait_ticks = 0;    // bound on one in-kernel wait of a sweep, s_memrealtime ticks
   int cus = 1;                          // compute units of the device
   size_t base_bytes = 0;                // bytes of the buffers above

@@ -54,7 +54,8 @@ struct SweepArgs {
   double* X;                   // first column of the group
   double* vec;                 // (products + 1) vectors of b x R (backward: two partial vectors each)
   unsigned* claims;            // seats: nonzero once a workgroup has taken it
-  int* err;
+  int* fail;                   // a wait of this launch has given up
+  int* err;                    // the same in host memory, set until the host has read it
   unsigned long long spin_ticks;
   int n, b, a, ldx, nr;        // nr <= R right-hand sides
   int parts;                   // work items per product
@@ -251,9 +252,10 @@ __device__ __forceinline__ void sweep_stage(const SweepArgs& p, SweepLds<R, U, T
   }
 }
 
-// Bound on a wait of a thread: it ends, with err, after spin_ticks, or once
-// another workgroup has raised err (looked at after 10 ms: polled by everyone from
-// the start, that one word would be a hot spot).
+// Bound on a wait of a thread: it ends for good, with fail and err, after
+// spin_ticks, or once another workgroup has raised fail (looked at after 10 ms:
+// polled by everyone from the start, that one word would be a hot spot).  What is
+// missing then stays kPending, a NaN, and spreads through what follows.
 struct SweepWait {
   const SweepArgs& p;
   unsigned long long t0 = 0;
@@ -261,10 +263,10 @@ struct SweepWait {
     __builtin_amdgcn_s_sleep(1);
     const unsigned long long now = __builtin_amdgcn_s_memrealtime();
     if (t0 == 0) t0 = now;
-    if (now - t0 < kPatience) return true;
-    if (__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0) return false;
-    if (now - t0 < p.spin_ticks) return true;
-    __hip_atomic_fetch_or(p.err, 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (now - t0 < p.spin_ticks)
+      return now - t0 < kPatience || __hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0;
+    __hip_atomic_store(p.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(p.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return false;
   }
 };
@@ -453,7 +455,7 @@ __global__ void __launch_bounds__(kSweepThreads + 64 * NP, 4) k_sweep(SweepArgs 
   else sweep_worker<R, U, T, NP>(p, l, stages, own);
 }
 
-// Before a sweep: the hand-over vectors (vector 0: the first block of the
+// Before a sweep: its fail word, the hand-over vectors (vector 0: the first block of the
 // sweep, the others kPending) and the claims, and before a backward
 // sweep x_a = T^-T y_a of all right-hand sides (`tip` > 0: their number), in
 // place.
@@ -463,6 +465,7 @@ __global__ void __launch_bounds__(BTA_THREADS) k_sweep_init(SweepArgs p, const d
                                                            const double* tinv, int tip) {
   const int group = blockIdx.y;
   if (blockIdx.x == 0 && group == 0) {
+    if (threadIdx.x == 0) *p.fail = 0;
     const int a = p.a, per = tip > 0 ? BTA_THREADS / a : 1;
     for (int c0 = 0; c0 < tip; c0 += per) {
       const int q = threadIdx.x / per, rc = c0 + threadIdx.x % per;
@@ -790,7 +793,8 @@ int potrs_enqueue(Workspace& ws, const double* L, const double* B, int n, int b,
   p.X = rhs;
   p.vec = nullptr;
   p.claims = nullptr;
-  p.err = ws.err;
+  p.fail = ws.sweep_fail;
+  p.err = ws.solve_err;
   p.spin_ticks = ws.wait_ticks;
   p.n = n;
   p.b = b;

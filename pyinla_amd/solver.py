@@ -159,7 +159,7 @@ class SerinvSolver:
         _lib.check(self.lib.bta_ws_set_option(self._ws, 7, 1 if on else 0), "set_option")
 
     def status(self):
-        """(info, logdet, err) of the last factorization (synchronises)."""
+        """(info, logdet) of the last factorization (synchronises)."""
         info = C.c_int64()
         ld = C.c_double()
         err = C.c_int()
@@ -167,7 +167,7 @@ class SerinvSolver:
             _lib.check(self.lib.bta_ws_status(self._ws, C.byref(info), C.byref(ld), C.byref(err),
                                               _stream_ptr(self.device)), "bta_ws_status")
         if err.value:
-            raise _lib.BTALibraryError("in-kernel wait timed out during the factorization")
+            raise _lib.BTALibraryError("in-kernel wait timed out during the factorization or a triangular sweep after it")
         return int(info.value), float(ld.value)
 
     def load_blocks(self, D, L, B=None, T=None) -> None:
@@ -218,7 +218,8 @@ class SerinvSolver:
 
         ``rhs`` is a float64 torch tensor on the solver's device of shape (N,)
         or (N, nrhs), overwritten and returned; a numpy array is solved on the
-        device and written back in place.
+        device and written back in place.  Raises BTALibraryError (and leaves a
+        numpy ``rhs`` as it was) if a wait between the sweeps' workgroups timed out.
         """
         _check_sparsity(sparsity)
         tic = time.perf_counter()
@@ -242,6 +243,9 @@ class SerinvSolver:
                 _lib.check(self.lib.bta_potrs(self._ws, _ptr(D), _ptr(L), _ptr(B), _ptr(T), n, b, a,
                                               C.c_void_p(X.data_ptr()), nrhs, nrhs, trans, st), "bta_potrs")
         torch.cuda.synchronize(self.device)
+        err = C.c_int()
+        _lib.check(self.lib.bta_solve_status(self._ws, C.byref(err), st), "bta_solve_status")
+        _lib.check(err.value, "solve")
         self.t_solve += time.perf_counter() - tic
         if host is not None:
             host[...] = x.cpu().numpy().reshape(host.shape)
