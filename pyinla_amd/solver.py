@@ -320,8 +320,10 @@ class SerinvSolver:
 
     @staticmethod
     def _index_pair(rows, cols):
-        """Contiguous index arrays of one 4- or 8-byte integer type."""
+        """Contiguous index arrays of one length and one 4- or 8-byte integer type."""
         rows, cols = np.asarray(rows), np.asarray(cols)
+        if rows.ndim != 1 or rows.shape != cols.shape:
+            raise ValueError(f"row and column indices do not match: {rows.shape} and {cols.shape}")
         dt = np.int32 if rows.dtype == np.int32 and cols.dtype == np.int32 else np.int64
         return np.ascontiguousarray(rows, dtype=dt), np.ascontiguousarray(cols, dtype=dt)
 
