@@ -54,6 +54,17 @@ def bytes_potrs(n, b, a):
     return 16 * (n * b**2 + (n - 1) * b**2 + n * a * b + a**2)
 
 
+def class_kernel(cls, b, panel_launches, blocks):
+    """Kernels whose launches a timing class holds; the panel variants are told
+    apart by their launches for ``blocks`` blocks of edge ``b``."""
+    if cls == 0:
+        if panel_launches < blocks:
+            return "k_chain64"
+        return "k_panel_flow" if b > 64 and panel_launches == blocks else "k_panel_step"
+    return {1: "k_gemm_nt_sub / k_gemm_grouped", 2: "k_gemm_direct / k_gemm_grouped",
+            3: "k_sweep_solo" if b <= 64 else "k_sweep", 4: "rocblas_dgemm"}[cls]
+
+
 def parse():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -415,10 +426,9 @@ def main():
         ach = per_launch_flops / (avg_ms * 1e-3) / 1e12
         roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                 "frac": ach / PEAK_FP64_TFLOPS, "traffic": None}
-    roof["kernel"] = {0: "k_panel_flow" if flow else "k_panel_step", 1: "k_gemm_nt_sub", 2: "k_gemm_grouped",
-                      3: "k_sweep", 4: "rocblas_dgemm"}[dom]
-    # HBM bytes per launch of that kernel from the committed rocprofv3 PMC
-    # summary (FETCH_SIZE / WRITE_SIZE, scaled by a 1 GiB copy), if present
+    roof["kernel"] = class_kernel(dom, b, cnt[0], 2 * n)
+    # HBM bytes per launch from the committed rocprofv3 PMC summary (FETCH_SIZE /
+    # WRITE_SIZE, scaled by a 1 GiB copy), where the class is one kernel in it
     tr_path = ROOT / "profiles" / "pmc_traffic.json"
     if tr_path.exists():
         try:
