@@ -21,6 +21,7 @@
 
 #include "bta_internal.h"
 #include "../../include/pyinla_bta.h"
+#include "bta_batch_rule.h"
 #include "bta_blocks16.h"
 
 namespace bta {
@@ -786,58 +787,6 @@ static std::vector<int> helper_shares(const std::vector<int>& nT, int each) {
   return h;
 }
 
-// A block step in us, from lone and batched launches on MI355X: the chain takes
-// 15.2 us per tile column, a block 3.3 nT^3 us of one helper that has its CU to
-// itself and 4.5 of one that shares it.
-static double step_work(const std::vector<int>& nT) {
-  double w = 0.0;
-  for (const int t : nT) w += (double)t * t * t;
-  return w;
-}
-static double step_chain(const std::vector<int>& nT) { return 15.2 * *std::max_element(nT.begin(), nT.end()); }
-// One workgroup per CU is enough to keep the longest chain the bound (a second
-// one on some CUs makes those helpers late: b = 1600 with b = 100 4.3 ms per 10
-// blocks, 3.9 with one per CU).
-static bool step_fits_one(const std::vector<int>& nT, int cus) {
-  const int np = (int)nT.size(), h = cus / np - 1;
-  return h >= 1 && 3.3 * step_work(nT) <= step_chain(nT) * h * np;
-}
-static double step_time(const std::vector<int>& nT, int cus, int cap) {
-  if (step_fits_one(nT, cus)) return step_chain(nT);
-  return std::max(step_chain(nT), 4.5 * step_work(nT) / std::max(1, cap - 2 * (int)nT.size()));
-}
-
-// Problems per wave: the number that the estimate above says is fastest, by the
-// steps of all waves and 10 us per launch.  Chains side by side cost nothing
-// until the helpers are the bound.  Finite-difference stencil of 18 problems,
-// nt = 16, in ms as waves of 6, 9, 18: b = 120 5.5, 4.9, 4.4; b = 480 11.0, 9.8,
-// 8.4; b = 840 21.7, 20.0, 21.6.
-static int pick_lanes(const std::vector<ProbDesc>& ps, const std::vector<int>& order, int cus, int cap) {
-  const int np = (int)ps.size();
-  int best = 1;
-  double best_t = 0.0;
-  for (int nl = 1; nl <= std::min(np, FLOW_BATCH_MAX) && cap / nl - 1 >= 1; ++nl) {
-    double t = 0.0;
-    for (int w0 = 0; w0 < np; w0 += nl)
-      for (int i = 0; i < ps[order[w0]].n;) {  // longest first
-        std::vector<int> nts;
-        int until = 1 << 30;
-        for (int q = w0; q < std::min(np, w0 + nl); ++q)
-          if (i < ps[order[q]].n) {
-            nts.push_back(ps[order[q]].nT);
-            until = std::min(until, ps[order[q]].n);
-          }
-        t += (until - i) * (step_time(nts, cus, cap) + 10.0);
-        i = until;
-      }
-    if (nl == 1 || t < best_t) {
-      best = nl;
-      best_t = t;
-    }
-  }
-  return best;
-}
-
 int BatchPlan::build(const std::vector<ProbDesc>& ps, int panel_mode, int lanes, int delta, int near_div,
                      int device) {
   probs = ps;
@@ -858,7 +807,10 @@ int BatchPlan::build(const std::vector<ProbDesc>& ps, int panel_mode, int lanes,
     std::vector<int> order(np);
     for (int q = 0; q < np; ++q) order[q] = q;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ps[x].n > ps[y].n; });
-    const int nl = std::min(lanes > 0 ? std::min(lanes, np) : pick_lanes(ps, order, cus, cap), FLOW_BATCH_MAX);
+    std::vector<BatchShape> shapes;
+    for (const int q : order) shapes.push_back(BatchShape{ps[q].n, ps[q].nT});
+    const int nl = std::min(lanes > 0 ? std::min(lanes, np) : pick_lanes(shapes, FLOW_BATCH_MAX, cus, cap),
+                            FLOW_BATCH_MAX);
     if (cap / nl - 1 < 1) {
       flow = false;  // too many problems to give each a resident chain + helper
     } else {
