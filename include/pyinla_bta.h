@@ -191,7 +191,7 @@ int bta_logdet(bta_ws_t ws, const double* D, const double* T, int n, int b, int 
  * operand forms, operands loaded straight into registers (32x32 or 64x64
  * tiles) or staged through one LDS buffer (triangular products); 1 = 64x64
  * tiles through two LDS buffers with loads issued two K chunks ahead (slower
- * on MI355X: 470 us against 262 us for NN 2000^3; kept for comparison). */
+ * on MI355X: 354 us against 262 us for NN 2000^3; kept for comparison). */
 #define BTA_OPT_GEMM_KERNEL 9
 /* Persistent panel, block update D_{i+1} -= L_i L_i^T, B_{i+1} -= B_i L_i^T,
  * T -= B_i B_i^T: 1 = applied by each block's launch through helper tasks

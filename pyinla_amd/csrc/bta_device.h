@@ -75,19 +75,6 @@ __device__ __forceinline__ void lds_load_tile(double* __restrict__ s, const doub
   }
 }
 
-// Same, but store the transpose: s[c][r] = g[r][c].
-__device__ __forceinline__ void lds_load_tile_t(double* __restrict__ s, const double* __restrict__ g,
-                                                int64_t ld, int rows, int cols) {
-  const int c = threadIdx.x & 63;
-  const int r0 = threadIdx.x >> 6;
-#pragma unroll 4
-  for (int r = r0; r < 64; r += 4) {
-    double v = 0.0;
-    if (r < rows && c < cols) v = g[(int64_t)r * ld + c];
-    s[c * BTA_LDS_LD + r] = v;
-  }
-}
-
 // A 64x64 operand tile staged global -> registers -> LDS, so that the global
 // loads of the next K chunk are in flight while the current chunk is
 // multiplied.  The LDS layout is always s[i][k] (row i of op(X), column k).
@@ -308,17 +295,6 @@ __device__ __forceinline__ void st_sys(double* p, double v) {
 }
 __device__ __forceinline__ double ld_sys(const double* p) {
   return __hip_atomic_load(const_cast<double*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// A 64 x 64 accumulator tile to a contiguous 64 x 64 buffer with system-scope
-// stores.
-__device__ __forceinline__ void acc_store_sys(const TileAcc& t, double* __restrict__ g) {
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) st_sys(&g[acc_row(x, r) * 64 + acc_col(y)], t.c[x][y][r]);
 }
 
 // All threads call after their st_sys stores of the guarded data.

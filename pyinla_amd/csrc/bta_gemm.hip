@@ -281,8 +281,8 @@ namespace bta {
 // ------------------------------------------- 64x64 tiles, pipelined K loop
 //
 // Variant of the grouped GEMM (BTA_OPT_GEMM_KERNEL 1; measured slower on
-// MI355X than the single-buffered k_gemm_grouped above, 470 us against 395 us
-// for NN 2000^3, and kept for comparison).  K advances in chunks of 16; the
+// MI355X than the kernels above, NN 2000^3 354 us against 293 for k_gemm_grouped
+// and 262 for k_gemm_direct, and kept for comparison).  K advances in chunks of 16; the
 // A chunk (64 rows of op(A) x 16) is kept in LDS as sA[i][k] (odd stride 17)
 // and the B chunk (16 x 64 columns of op(B)) as sB[k][j] (stride 68), so the
 // MFMA operand reads of a wave (16 rows x 4 k) hit distinct banks.  Two LDS

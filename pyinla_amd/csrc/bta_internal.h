@@ -18,9 +18,9 @@ static constexpr unsigned long long kInfoNone = ~0ull;
 
 // Kernel classes for the optional event timing of bta_ws_set_timing.
 enum KernelClass : int {
-  KC_PANEL = 0,     // k_panel_step (tile-column factorization)
-  KC_UPDATE = 1,    // k_gemm_nt_sub (block updates D_{i+1}, B_{i+1}, T)
-  KC_GROUPED = 2,   // k_gemm_grouped (block inverses, selected inversion)
+  KC_PANEL = 0,     // k_panel_flow, k_panel_step or k_chain64 (factorization)
+  KC_UPDATE = 1,    // block updates of their own (k_gemm_nt_sub or a grouped launch)
+  KC_GROUPED = 2,   // grouped GEMMs (block inverses, selected inversion), k_chain64_selinv
   KC_GEMV = 3,      // triangular sweeps
   KC_BLAS = 4,      // rocBLAS dgemm of the selected inversion (Sigma_{i+1,i} products)
   KC_COUNT = 5

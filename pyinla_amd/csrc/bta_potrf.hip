@@ -626,12 +626,14 @@ int flow_alloc(Workspace& ws) {
 }
 
 // Whether the persistent panel applies the block update itself.  Measured on
-// MI355X (factorizations of Q_prior and Q_cond, ms per block, lone / pair on
-// two streams): b = 2000 (32 tile columns) in the panel 0.918 / 1.318, as a
-// GEMM after it 0.941 / 1.397; b = 4500 (71 tile columns) in the panel
-// 9.10 / 15.47, as a GEMM 7.46 / 14.16.  The helpers are the bound in both
-// cases: for wide panels the separate update (one large grouped GEMM) is the
-// cheaper way to do its share of the work.
+// MI355X, ms per block, lone factorization / pair on two streams:
+//   tile columns      32           41           47           57           71
+//   in the panel  0.54 /  0.87 1.02 / 2.09 1.72 / 3.44 3.03 / 6.59 6.19 / 15.1
+//   GEMM after it 0.68 /  1.10 1.06 / 2.16 1.71 / 3.21 2.95 / 5.76 5.74 / 12.3
+// The panels' helpers read their operands past L2, and the wider the panel the
+// more of them past the last-level cache as well; one large grouped GEMM then does
+// the update's share of the work for less.  (They cross near 46 columns alone and
+// 44 as a pair; 48 gives away 1 % and 7 % at 47.)
 static int flow_fold_of(const Workspace& ws, int b) {
   if (ws.flow_fold == 1 || ws.flow_fold == 2) return ws.flow_fold == 1;
   return (b + 63) / 64 <= 48;
