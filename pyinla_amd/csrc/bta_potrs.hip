@@ -18,13 +18,13 @@
 //
 // Measured on MI355X, us per product (2n of them in a sweep), forward /
 // backward, against one launch per product:
-//   b = 48            0.84 / 0.98   (7.1 / 6.2)   one workgroup, vectors in LDS
-//   b = 92            1.8 / 1.8     (7.2 / 7.4)
-//   b = 400           1.9 / 1.9     (7.3 / 8.7)
-//   b = 800           3.0 / 3.3     (8.6 / 11.1)
-//   b = 1600          5.2 / 6.1     (11.3 / 13.7) its bytes at 5 TB/s: 3.1
-//   b = 4500          27 / 37       (37 / 37)     its bytes at 5 TB/s: 24
-//   b = 800, 16 right-hand sides    7 / 9         (78 / 55)
+//   b = 48            0.63 / 0.89   (7.1 / 6.2)   one workgroup, vectors in LDS
+//   b = 92            1.3 / 1.4     (7.2 / 7.4)
+//   b = 400           1.3 / 1.5     (7.3 / 8.7)
+//   b = 800           2.3 / 2.8     (8.6 / 11.1)
+//   b = 1600          4.1 / 5.6     (11.3 / 13.7) its bytes at 5 TB/s: 3.1
+//   b = 4500          25 / 34       (37 / 37)     its bytes at 5 TB/s: 24
+//   b = 800, 8 right-hand sides     3.8 / 3.8; 16 6.4 on average (78 / 55)
 #include <algorithm>
 
 #include "bta_internal.h"
@@ -42,7 +42,7 @@ typedef __attribute__((address_space(1))) d2 gd2;
 // of an FP64 operation, and those quiet NaNs, so no value can equal it.
 constexpr unsigned long long kPending = 0x7FF4C0DEC0DE0001ull;
 // Largest block swept by a single workgroup: one CU reads its matrices at 25 to
-// 32 GB/s, at b = 92 (68 KB) 2.1 / 2.7 us per product against 1.8 / 1.8 with the
+// 32 GB/s, at b = 92 (68 KB) 2.1 / 2.7 us per product against 1.3 / 1.4 with the
 // hand-over.
 constexpr int kSolo = 64;
 constexpr int kSoloThreads = 512;   // kSolo x 8
@@ -819,9 +819,9 @@ int potrs_enqueue(Workspace& ws, const double* L, const double* B, int n, int b,
     // passes take the least (one of 1, 4 and 8 is as 1 : 1.6 : 2.5).  Measured on
     // MI355X, ms for 1, 4, 8, 16, 32 right-hand sides, in brackets with one
     // group of 4 or 8 after the other:
-    //   n = 50, b = 92     0.37 0.37 0.38 0.41 0.79   (0.36 0.62 0.95 1.87 3.72)
-    //   n = 40, b = 300    0.32 0.34 0.61 0.64 0.99   (0.32 0.60 0.91 1.80 3.57)
-    //   n = 40, b = 800    0.50 0.77 0.78 1.24 2.51   (0.50 0.79 1.22 2.44 4.92)
+    //   n = 50, b = 92     0.31 0.32 0.32 0.35 0.68   (0.36 0.62 0.95 1.87 3.72)
+    //   n = 40, b = 300    0.28 0.29 0.52 0.54 0.81   (0.32 0.60 0.91 1.80 3.57)
+    //   n = 40, b = 800    0.45 0.68 0.67 1.02 2.08   (0.50 0.79 1.22 2.44 4.92)
     const double* x0 = rhs + (trans ? (int64_t)(n - 1) * b * ldrhs : 0);
     const int room = std::max(1, ws.cus / std::min((b + 7) / 8, ws.cus));
     auto slots = [&](int R) { return (int)std::min<size_t>(ws.work_doubles / group_doubles(n, b, R), room); };
